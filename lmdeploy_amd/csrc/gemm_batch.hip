@@ -136,12 +136,14 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     // Patch: row r is 128 bytes, its 16-byte chunk k at position k ^ f(r), f(r) = (r & 7) ^ (r >> 3 & 1): the 16 lanes that
     // read one chunk of 16 rows then touch every bank group equally, whether LDS serves 8 or 16 lanes per clock.
     // Load i brings rows 8i .. 8i + 7; the swizzle is applied by which chunk each lane fetches.
-    // (lane offsets are biased by 3 KiB - the load's position in its group of four, which load_lds adds to both addresses)
+    // (Lane offsets are biased by 3 KiB - the load's position in its group of four, which load_lds adds to both addresses.
+    // They count from the block's first token: at most 16 H - 1 rows of X and the bias, which 32 bits hold wherever they
+    // hold X; from the first row of X the bias would carry the last rows of a 4 GiB X past them.)
     uint32_t x_off[NX];
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
         const int r = 8 * i + (lane >> 3);
-        x_off[i]    = (uint32_t)min(t0 + r, T - 1) * (uint32_t)(K * 2) + (uint32_t)(((lane & 7) ^ (r & 7) ^ (r >> 3 & 1)) * 16 + (3 - i % 4) * 1024);
+        x_off[i]    = (uint32_t)min(r, T - 1 - t0) * (uint32_t)(K * 2) + (uint32_t)(((lane & 7) ^ (r & 7) ^ (r >> 3 & 1)) * 16 + (3 - i % 4) * 1024);
     }
     const uint32_t patch = __builtin_amdgcn_readfirstlane(lds_addr(smem) + (uint32_t)(wave * 2 * kPatch));
     uint32_t       xr[2];  // fragment of chunk j of a patch: row c, chunk 4j + b
@@ -152,7 +154,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     const int64_t w_step = (int64_t)NT * (kWaves * 1024), q_step = (int64_t)NQ * N * (kWaves * 4);
     const char*   wp = reinterpret_cast<const char*>(p.A) + ((int64_t)g0 * NT + col0) * 1024;
     const char*   qp = reinterpret_cast<const char*>(p.Q) + ((int64_t)g0 * NQ * N + col0 * kTileN) * 4;
-    const char*   xp = reinterpret_cast<const char*>(p.X) + (int64_t)g0 * 256 - 3072;
+    const char*   xp = reinterpret_cast<const char*>(p.X) + (int64_t)t0 * K * 2 + (int64_t)g0 * 256 - 3072;
 
     struct Stage {
         u32x4_t  w[R];
@@ -442,7 +444,8 @@ bool batch_feasible(const BatchConfig& cf, int N, int T, int K, size_t ws_bytes,
 {
     if (N <= 0 || T <= 0 || K <= 0 || N % kTileN != 0 || K % kGroup != 0) return false;
     if (!width_exists(cf.r, cf.h) || N / kTileN < cf.r) return false;
-    if ((int64_t)T * K * 2 + 4096 >= (1ll << 32)) return false;  // 32-bit per-lane offsets into X, biased by 3 KiB
+    // the bound of the strips, which run on this kernel up to kWidestBatchStrip tiles wide (its own offsets reach one block)
+    if ((int64_t)T * K * 2 >= (1ll << 32)) return false;
     const int64_t tiles = (int64_t)((N / kTileN + cf.r - 1) / cf.r) * ((T + 16 * cf.h - 1) / (16 * cf.h));
     if (cf.splits > 1 && (K / kGroup < cf.splits || tiles > cnt_len || (int64_t)batch_scratch_bytes(cf, N, T) > (int64_t)ws_bytes)) return false;
     return cf.splits >= 1 && tiles * cf.splits < (1ll << 31);
