@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libw4a16.so")
 
-SOURCES = ["api.cpp", "repack.hip", "static_scratch.hip", "probe.hip", "gemm_decode.hip", "gemm_strip.hip", "gemm_strip_groups.hip",
+SOURCES = ["api.cpp", "rounding_domain.cpp", "repack.hip", "static_scratch.hip", "probe.hip", "gemm_decode.hip", "gemm_strip.hip", "gemm_strip_groups.hip",
            "gemm_sequence.hip", "gemm_prefill.hip", "gemm_batch.hip", "gemm_tile_g128.hip", "gemm_tile_g64.hip", "gemm_tile_g32.hip"]
 
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 instructions for this target.

@@ -118,6 +118,8 @@ bool algo_feasible(int id, int N, int T, int K, const Scratch& lim);
 size_t algo_scratch_bytes(int id, int N, int T, int K, const Scratch& lim);
 // heuristic choice (the counterpart of Estimate) for nq quantisation groups per weight tile; -1 if nothing is feasible
 int algo_pick(int nq, int N, int T, int K, const Scratch& lim);
+// whether a size's scales multiply sums in fp32, and not the weights, which rounds them (rounding_domain.cpp); `lim` as in algo_pick
+bool scales_in_fp32(int nq, int N, int T, int K, const Scratch& lim);
 // workgroups the launch would use
 int algo_grid(int id, int N, int T, int K, const Scratch& sc);
 hipError_t algo_launch(int id, int nq, const GemmArgs& a, const Scratch& sc, hipStream_t st);
