@@ -116,8 +116,9 @@ const Algo& algo_at(int id);
 bool algo_feasible(int id, int N, int T, int K, const Scratch& lim);
 // bytes of partial-tile scratch the launch would use (0: the kernel needs neither workspace nor counters)
 size_t algo_scratch_bytes(int id, int N, int T, int K, const Scratch& lim);
-// heuristic choice (the counterpart of Estimate) for nq quantisation groups per weight tile; -1 if nothing is feasible
-int algo_pick(int nq, int N, int T, int K, const Scratch& lim);
+// heuristic choice (the counterpart of Estimate) for nq quantisation groups per weight tile, among the kernels that do not round
+// weights if so asked; -1 if nothing is feasible
+int algo_pick(int nq, int N, int T, int K, const Scratch& lim, bool unrounded = false);
 // whether a size's scales multiply sums in fp32, and not the weights, which rounds them (rounding_domain.cpp); `lim` as in algo_pick
 bool scales_in_fp32(int nq, int N, int T, int K, const Scratch& lim);
 // workgroups the launch would use

@@ -82,3 +82,26 @@ def test_sizes_that_were_never_rounded_without_a_workspace(tm, K, N, T):
         g.replay()
         torch.cuda.synchronize()
         check(C, want, rounded, (K, N, T))
+
+
+@pytest.mark.parametrize("gs", [64, 32])
+@pytest.mark.parametrize("T", [33, 300, 1000])
+def test_small_groups_with_outputs_of_four_bytes_of_alignment(tm, gs, T):
+    """The rounding tile of group sizes 64 and 32 never took such outputs; SiLU pairs always fitted."""
+    K, N = 4096, 4096
+    A, Q, X, want, rounded = problem(tm, K, N, T, gs)
+    buf = torch.zeros(2 * T * N + 8, dtype=torch.float16, device="cuda")
+    low, high = buf[2:2 + T * N].view(T, N), buf[4 + T * N:4 + 2 * T * N].view(T, N)
+    assert low.data_ptr() % 8 == 4 and high.data_ptr() % 8 == 0
+    aligned = torch.zeros((T, N), dtype=torch.float16, device="cuda")
+    for kind, C, R in ((0, low, None), (2, low, high), (2, aligned, low)):
+        C.fill_(float("nan"))
+        if R is not None:
+            R.zero_()
+        tm.GemmS4F16().Run(C, A, X, Q, N, T, K, gs, kind, residual=R)
+        check(C, want, rounded, (gs, T, kind))
+        if R is not None:
+            R.zero_()
+        C.fill_(float("nan"))
+        tm.gemm_static(C, A, X, Q, N, T, K, gs, kind, residual=R)
+        check(C, want, rounded, (gs, T, kind, "static"))
