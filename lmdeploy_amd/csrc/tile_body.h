@@ -86,6 +86,17 @@ __device__ __forceinline__ void lds_read128(half8_t& dst, uint32_t addr)
 {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
+// g / (1 + exp(-g)) with the quotient rounded as a division rounds it: the approximate quotient and one correction by its exact
+// remainder (Markstein), special cases by the instruction that ends the compiler's division too.  Without the scaling that
+// a division of any two numbers needs: the denominator is at least one, and where its reciprocal is no longer a normal
+// number the result is zero in fp16.  The scaling goes through VCC, one quotient after the other, and a wave of this kernel
+// has its SIMD to itself: a 7B layer at 2048 tokens takes 714 us with `/`, 711 with this and 707 with the reciprocal alone, which
+// rounds one half in thirty thousand differently from the other kernels.
+__device__ __forceinline__ float silu_quotient(float g)
+{
+    const float d = 1.f + __expf(-g), r = __builtin_amdgcn_rcpf(d), q = g * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, g), r, q), d, g);
+}
 __device__ __forceinline__ uint64_t pack2(float a, float b)
 {
     return (uint64_t)__builtin_bit_cast(uint32_t, a) | ((uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
@@ -464,7 +475,7 @@ tile_kernel(uint16_t* __restrict__ C, const u32x4_t* __restrict__ A, const uint1
                     for (int e = 0; e < 2; ++e) {
                         const half2_t gu = as_half2(o[2 * i + e]);
                         const float   ga = (float)gu[0], up = (float)gu[1];
-                        h[e] = (half_t)(ga * __builtin_amdgcn_rcpf(1.f + __expf(-ga)) * up);
+                        h[e] = (half_t)(silu_quotient(ga) * up);
                     }
                     r[i] = as_u32(half2_t{h[0], h[1]});
                 }
