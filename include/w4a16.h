@@ -108,8 +108,9 @@ int w4a16_gemm(w4a16_handle* h, void* C, const void* A, const void* X, const voi
  * tiles) fails with W4A16_ESCRATCH.  It calls no allocating routine; the buffer's device address
  * is looked up (hipGetSymbolAddress) by the first call on a device or by w4a16_create.  All calls
  * on one GPU share the one buffer: calls that can overlap on the GPU (different streams, or
- * different threads) race, so order them on one stream.  The counts of a launch carry a tag of their own, so that
- * what a race or an abandoned launch leaves in the counters does not concern the launches after it. */
+ * different threads) race, so order them on one stream.  What a race or an abandoned launch leaves in the counters does
+ * not concern the launches after it: the counts of a launch carry a tag of their own, and a launch that is recorded
+ * into a graph, whose replays all carry the same one, clears the counters it will use with a small kernel before it. */
 int w4a16_gemm_static(void* C, const void* A, const void* X, const void* Q, const void* R, int n_out, int tokens,
                       int k, int group_size, int epilogue, int algo_id, void* stream);
 

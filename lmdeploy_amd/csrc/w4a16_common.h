@@ -158,10 +158,10 @@ __device__ __forceinline__ void spread_q(uint32_t x, uint32_t* q)
 }
 
 // Split K: a workgroup announces that its partial tile is complete; true for the last of `splits`, which leaves the counter
-// at zero for the next launch.  epoch 0: the counters belong to a handle, nobody else touches them.  Otherwise they are
-// shared by every caller on the GPU: a count tagged with another launch's epoch - left behind by launches that
-// overlapped against the rules - is taken for zero, so that one misuse does not spoil the launches after it, and no
-// launch has to be preceded by one that clears them.  (A graph's replays share an epoch; each leaves zeros.)
+// at zero for the next launch.  epoch 0: the counters belong to a handle, which nobody else touches, or were cleared right before
+// this launch.  Otherwise they are shared by every caller on the GPU and start from whatever is there: a count tagged with
+// another launch's epoch - left behind by launches that overlapped against the rules - is taken for zero, so that one misuse
+// does not spoil the launches after it and none of them has to be preceded by one that clears the counters.
 __device__ __forceinline__ bool arrive_last(int* counter, int splits, int epoch)
 {
     if (epoch == 0) {

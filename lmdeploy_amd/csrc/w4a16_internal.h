@@ -130,6 +130,8 @@ hipError_t algo_launch(int id, int nq, const GemmArgs& a, const Scratch& sc, hip
 constexpr size_t kStaticCounters       = 4096;
 constexpr size_t kStaticWorkspaceBytes = 8u << 20;
 hipError_t static_scratch(Scratch* out);
+// before a launch that uses `n` of its counters: sets the tag, and clears them where the launch is being recorded into a graph
+hipError_t prepare_static_counters(Scratch* sc, int n, hipStream_t st);
 
 hipError_t launch_convert(uint32_t* A_dst, uint32_t* Q_dst, const uint32_t* A_src, const uint16_t* scales,
                           const uint32_t* qzeros, int m, int k, int group, hipStream_t st);
