@@ -240,6 +240,32 @@ def _mfma_hazards(name: str, lines: List[Tuple[int, str]]) -> List[str]:
     return out
 
 
+_M0_WRITE = re.compile(r"^(?!s_cmp|s_bitcmp)\S+\s+m0\b")
+
+
+def _m0_hazards(name: str, lines: List[Tuple[int, str]]) -> List[str]:
+    """A direct-to-LDS load from inline assembly takes its LDS address from M0.  Where an assembly statement does not set M0
+    before such a load, it relies on an earlier statement's value, which the compiler does not know to be in use: then
+    no compiler-generated instruction of the function may write M0."""
+    borrowed, writes, in_asm, is_set = False, [], False, False
+    for ln, raw in lines:
+        s = raw.strip()
+        if s.startswith(";;#ASMSTART"):
+            in_asm, is_set = True, False
+            continue
+        if s.startswith(";;#ASMEND"):
+            in_asm = False
+            continue
+        code = raw.split(";")[0].strip()
+        if in_asm:
+            is_set = is_set or _M0_WRITE.match(code) is not None
+            borrowed = borrowed or ("_lds_" in code and not is_set)
+        elif _M0_WRITE.match(code):
+            writes.append((ln, code))
+    return ["%s: line %d writes M0, which an assembly statement sets for loads in later ones: %s" % (name, ln, code)
+            for ln, code in writes if borrowed]
+
+
 def lint(asm_text: str, only_if_name_has: str = "kernel") -> List[str]:
     """Returns one message per violation (empty list: clean)."""
     out: List[str] = []
@@ -258,6 +284,7 @@ def lint(asm_text: str, only_if_name_has: str = "kernel") -> List[str]:
             cur.append((ln, raw))
     for name, lines in funcs:
         out.extend(_mfma_hazards(name, lines))
+        out.extend(_m0_hazards(name, lines))
         blocks = _parse(lines)
         index = {b[0]: k for k, b in enumerate(blocks)}
         entry: List[Dict[int, int]] = [None] * len(blocks)  # type: ignore

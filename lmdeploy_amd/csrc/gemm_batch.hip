@@ -71,12 +71,12 @@ __device__ __forceinline__ void load_lds(uint32_t lds, const uint32_t* voff, con
                      "global_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, %4 offset:3072"
                      :
                      : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(sbase), "s"(lds)
-                     : "memory");
+                     : "memory", "m0");
     else
         asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024"
                      :
                      : "v"(voff[0]), "v"(voff[1]), "s"(sbase), "s"(lds)
-                     : "memory");
+                     : "memory", "m0");
 }
 
 // wait until at most N LDS reads are in flight; the fragments named are complete then

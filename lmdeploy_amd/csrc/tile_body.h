@@ -54,14 +54,15 @@ __device__ __forceinline__ void gload32(uint32_t& dst, uint32_t voff, const void
 // Global memory straight into LDS: lane l's 16 bytes land at lds_base + 16 l.  The LDS base travels
 // in M0; written here (rather than through the builtin) so that the address is a scalar base
 // plus a 32-bit lane offset instead of a 64-bit lane address, which costs a register pair and an
-// add per request.
+// add per request.  One value serves several requests, each a statement of its own: the build's assembly check
+// verifies that nothing else writes M0 in a kernel that relies on this.
 __device__ __forceinline__ uint32_t lds_addr(const void* p)
 {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)(p);
 }
 __device__ __forceinline__ void set_m0(uint32_t v)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(v) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(v) : "memory", "m0");
 }
 template<int OFF>
 __device__ __forceinline__ void gload_lds128_m0(uint32_t voff, const void* sbase)

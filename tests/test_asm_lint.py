@@ -94,3 +94,15 @@ def test_lds_reads_are_waited_for_by_count():
     assert lint(asm) == []
     asm = HEAD + read % (0, 3) + read % (4, 7) + "\ts_waitcnt lgkmcnt(1)\n\tv_mov_b32_e32 v20, v5\n" + TAIL
     assert len(lint(asm)) == 1
+
+
+def test_m0_written_by_the_compiler_where_loads_rely_on_it_is_reported():
+    put = "\t;;#ASMSTART\n\ts_mov_b32 m0, s5\n\ts_nop 0\n\t;;#ASMEND\n"
+    dma = "\t;;#ASMSTART\n\tglobal_load_lds_dwordx4 v40, s[2:3] offset:1024\n\t;;#ASMEND\n"
+    both = "\t;;#ASMSTART\n\ts_mov_b32 m0, s5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 v40, s[2:3]\n\t;;#ASMEND\n"
+    other = "\ts_mov_b32 m0, s9\n"
+    assert lint(HEAD + put + dma + dma + TAIL) == []
+    assert lint(HEAD + both + other + both + TAIL) == []                # (every statement sets its own)
+    assert lint(HEAD + put + dma + "\ts_cmp_eq_u32 m0, s9\n" + dma + TAIL) == []
+    msgs = lint(HEAD + put + dma + other + dma + TAIL)
+    assert len(msgs) == 1 and "writes M0" in msgs[0]
