@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     const int64_t w_step = (int64_t)NT * (kWaves * 1024), q_step = (int64_t)NQ * N * (kWaves * 4);
     const char*   wp = reinterpret_cast<const char*>(p.A) + ((int64_t)g0 * NT + col0) * 1024;
     const char*   qp = reinterpret_cast<const char*>(p.Q) + ((int64_t)g0 * NQ * N + col0 * kTileN) * 4;
-    const char*   xp = reinterpret_cast<const char*>(p.X) + (int64_t)t0 * K * 2 + (int64_t)g0 * 256 - 3072;
+    const char*   xp = reinterpret_cast<const char*>(p.X) + (uint32_t)t0 * ((uint32_t)K * 2) + (int64_t)g0 * 256 - 3072;
 
     struct Stage {
         u32x4_t  w[R];
