@@ -138,29 +138,14 @@ hipError_t launch_r(int tp, int depth, const StripParams& p, dim3 grid, size_t l
 
 constexpr int kInPasses = 3;  // value of `per_cu` that asks for one workgroup per CU walking several strips in turn
 
-// `per_cu` strips per CU are aimed for; more if a strip would otherwise be wider than the limit.
-// block_t = tokens per workgroup: 16 (activation rows padded down to 4 or 8 for fewer tokens) or 32.
-// Compute units of the current device (the strips are dealt to that many workgroups, or a multiple): asked
-// once per device; 256, MI355X's count, where no device can be asked.
-int device_cus()
-{
-    static std::atomic<int> cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return kNumCU;
-    int n = cached[dev].load(std::memory_order_relaxed);
-    if (n > 0) return n;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = kNumCU;
-    cached[dev].store(n, std::memory_order_relaxed);
-    return n;
-}
-
 }  // namespace
 
-StripPlan strip_plan(int per_cu, int block_t, int N, int T, int K)
+// `per_cu` strips for each of `cus` CUs are aimed for; more if a strip would otherwise be wider than the limit.
+// block_t = tokens per workgroup: 16 (activation rows padded down to 4 or 8 for fewer tokens) or 32.
+StripPlan strip_plan(int cus, int per_cu, int block_t, int N, int T, int K)
 {
-    const int cus = device_cus();
     StripPlan pl{};
-    if (N <= 0 || K <= 0 || T <= 0 || N % kTileN != 0 || K % kGroup != 0 || per_cu < 1) return pl;
+    if (N <= 0 || K <= 0 || T <= 0 || N % kTileN != 0 || K % kGroup != 0 || per_cu < 1 || cus < 1) return pl;
     if (block_t != 16 && block_t != 32) return pl;
     if (block_t == 32 && T <= 16) return pl;  // the 16-token kernel covers these
     const int NT   = N / kTileN;
@@ -193,25 +178,25 @@ StripPlan strip_plan(int per_cu, int block_t, int N, int T, int K)
     return pl;
 }
 
-bool strip_feasible(int per_cu, int block_t, int N, int T, int K)
+bool strip_feasible(int cus, int per_cu, int block_t, int N, int T, int K)
 {
-    return strip_plan(per_cu, block_t, N, T, K).ok;
+    return strip_plan(cus, per_cu, block_t, N, T, K).ok;
 }
 
-int strip_grid(int per_cu, int block_t, int N, int T, int K)
+int strip_grid(int cus, int per_cu, int block_t, int N, int T, int K)
 {
-    const StripPlan pl = strip_plan(per_cu, block_t, N, T, K);
+    const StripPlan pl = strip_plan(cus, per_cu, block_t, N, T, K);
     return pl.strips * ((T + block_t - 1) / block_t);  // (workgroups)
 }
 
-int strip_width(int per_cu, int block_t, int N, int T, int K)
+int strip_width(int cus, int per_cu, int block_t, int N, int T, int K)
 {
-    return strip_plan(per_cu, block_t, N, T, K).rmax;
+    return strip_plan(cus, per_cu, block_t, N, T, K).rmax;
 }
 
-hipError_t strip_launch(int per_cu, int block_t, const GemmArgs& a, hipStream_t st)
+hipError_t strip_launch(int cus, int per_cu, int block_t, const GemmArgs& a, hipStream_t st)
 {
-    const StripPlan pl = strip_plan(per_cu, block_t, a.N, a.T, a.K);
+    const StripPlan pl = strip_plan(cus, per_cu, block_t, a.N, a.T, a.K);
     if (!pl.ok) return hipErrorInvalidValue;
     const int   tp = block_t == 32 ? 32 : (a.T <= 4 ? 4 : (a.T <= 8 ? 8 : 16));
     const int   h  = tp > 16 ? tp / 16 : 1;

@@ -71,9 +71,9 @@ hipError_t launch_q(const StripPlan& pl, int tp, const StripParams& p, dim3 grid
 
 }  // namespace
 
-hipError_t strip_groups_launch(int nq, int per_cu, const GemmArgs& a, hipStream_t st)
+hipError_t strip_groups_launch(int nq, int cus, int per_cu, const GemmArgs& a, hipStream_t st)
 {
-    const StripPlan pl = strip_plan(per_cu, 16, a.N, a.T, a.K);
+    const StripPlan pl = strip_plan(cus, per_cu, 16, a.N, a.T, a.K);
     if (!pl.ok || (nq != 2 && nq != 4)) return hipErrorInvalidValue;
     const int   tp = a.T <= 4 ? 4 : (a.T <= 8 ? 8 : 16);
     StripParams p{a.C, reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.R, a.N, a.T, a.K, pl.base, pl.rem,

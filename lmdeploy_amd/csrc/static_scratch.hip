@@ -25,6 +25,7 @@ static __device__ __align__(256) unsigned char scratch[kStaticBytes];
 
 std::mutex     g_mutex;
 unsigned char* g_ptr[kMaxDevices];  // device address of `scratch` on each device, null until looked up
+int            g_cus[kMaxDevices];  // and the device's compute units
 
 // A launch made at once tags its counts with a number of its own (arrive_last); zero, a handle's tag, is that of launches
 // recorded into a graph.
@@ -52,9 +53,12 @@ hipError_t static_scratch(Scratch* out)
             e       = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
             if (e != hipSuccess) return e;
             if (!p) return hipErrorInvalidSymbol;
+            e = hipDeviceGetAttribute(&g_cus[dev], hipDeviceAttributeMultiprocessorCount, dev);
+            if (e != hipSuccess) return e;
             g_ptr[dev] = static_cast<unsigned char*>(p);
         }
-        ptr = g_ptr[dev];
+        ptr      = g_ptr[dev];
+        out->cus = g_cus[dev];
     }
     out->cnt      = reinterpret_cast<int*>(ptr);
     out->cnt_len  = (int)kStaticCounters;

@@ -81,6 +81,7 @@ struct Scratch {
     int*   cnt;
     int    cnt_len;
     int    epoch;  // tag of this launch's counts where the counters are shared, else 0 (arrive_last)
+    int    cus;    // compute units of the device that all this is on, which the strips are dealt to and the prices counted in
 };
 constexpr int kEpochShift = 12;  // a counter word: the epoch above, up to 4095 arrivals below
 
@@ -164,14 +165,14 @@ size_t     decode_scratch_bytes(const DecodeConfig& cf, int N, int T, int K, siz
 int        decode_grid(const DecodeConfig& cf, int N, int T, int K, size_t ws_bytes, int cnt_len);
 hipError_t decode_launch(const DecodeConfig& cf, const GemmArgs& a, const Scratch& sc, hipStream_t st);
 
-// decode kernels, strip decomposition (gemm_strip.hip); block_t = tokens per workgroup, 16 or 32
-bool       strip_feasible(int per_cu, int block_t, int N, int T, int K);
-int        strip_grid(int per_cu, int block_t, int N, int T, int K);
-int        strip_width(int per_cu, int block_t, int N, int T, int K);  // column tiles of the widest strip
-hipError_t strip_launch(int per_cu, int block_t, const GemmArgs& a, hipStream_t st);
+// decode kernels, strip decomposition (gemm_strip.hip); block_t = tokens per workgroup, 16 or 32, dealt to `cus` CUs
+bool       strip_feasible(int cus, int per_cu, int block_t, int N, int T, int K);
+int        strip_grid(int cus, int per_cu, int block_t, int N, int T, int K);
+int        strip_width(int cus, int per_cu, int block_t, int N, int T, int K);  // column tiles of the widest strip
+hipError_t strip_launch(int cus, int per_cu, int block_t, const GemmArgs& a, hipStream_t st);
 // the same for group sizes 64 and 32 (nq = 2, 4 quantisation groups per 128-row weight tile; gemm_strip_groups.hip), 16 tokens
 // per workgroup
-hipError_t strip_groups_launch(int nq, int per_cu, const GemmArgs& a, hipStream_t st);
+hipError_t strip_groups_launch(int nq, int cus, int per_cu, const GemmArgs& a, hipStream_t st);
 // How the column tiles are dealt out: `strips` workgroups, strips of base tiles (the first rem: one more), rmax wide at most.
 struct StripPlan {
     int  strips, base, rem, rmax;
@@ -180,7 +181,7 @@ struct StripPlan {
     bool narrow;  // sixteen waves per workgroup
     bool ok;
 };
-StripPlan strip_plan(int per_cu, int block_t, int N, int T, int K);
+StripPlan strip_plan(int cus, int per_cu, int block_t, int N, int T, int K);
 
 // The 32-token strips: up to this many column tiles wide, the batch kernel's way of feeding the activations is ahead of
 // the strip kernel's (7B qkv, strips of three, at 20 tokens 14.6 -> 9.6 us, o 6.3 -> 5.6); wider ones stream weights most

@@ -14,7 +14,7 @@ TAG_SHIFT = 12      # a counter word: the launch's tag above, arrivals below (w4
 class Scratch(ctypes.Structure):
     """w4a16::Scratch."""
     _fields_ = [("ws", ctypes.c_void_p), ("ws_bytes", ctypes.c_size_t), ("cnt", ctypes.c_void_p), ("cnt_len", ctypes.c_int),
-                ("epoch", ctypes.c_int)]
+                ("epoch", ctypes.c_int), ("cus", ctypes.c_int)]
 
 
 def scratch(lib):
