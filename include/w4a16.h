@@ -49,7 +49,8 @@ typedef struct w4a16_metric {
     int   kind;        /* 0 = decode kernel (column blocks), 1 = MFMA tiles, 2 = decode kernel (strips), 3 = batch kernel */
     int   tile_n;      /* output features per workgroup                         */
     int   tile_t;      /* tokens per workgroup                                  */
-    int   slices;      /* decode: K slices (wave groups) per workgroup; MFMA tiles and batch: workgroups that split K */
+    int   slices;      /* decode: K slices (wave groups) per workgroup, times the workgroups that split K
+                           where their number is the configuration's own; MFMA tiles and batch: workgroups that split K */
     int   grid;        /* workgroups launched                                   */
     float ms;          /* total time of `count` launches, +inf if not feasible  */
     int   count;       /* number of timed launches                              */

@@ -59,7 +59,7 @@ struct Algo {
     Family       family;
     int          tile_n;   // output features per workgroup
     int          tile_t;   // tokens per workgroup
-    int          slices;   // decode: K slices per workgroup; MFMA tiles and batch: K splits across workgroups
+    int          slices;   // as w4a16_metric reports them
     int          param;    // prefill: variant index; strips: strips per CU aimed for
     DecodeConfig dc;       // decode only
     BatchConfig  bc;       // batch only

@@ -86,3 +86,14 @@ def test_four_bytes_of_alignment(tm, T, N):
     tm.GemmS4F16().Run(C, A, X, Q, N, T, K, 128)
     assert ((C.float() - want).abs() <= allowed).all()
     assert (buf[:2] == 0).all() and (buf[2 + T * N:] == 0).all()
+
+
+def test_column_blocks_of_the_batch_kernel_report_their_split(tm):
+    """Eight waves of one, two or four workgroups share out K: three configurations, told apart by their slices."""
+    gemm, T, N, K = tm.GemmS4F16(), 16, 1024, 4096
+    A, Q, X, want, allowed = problem(tm, K, N, T, 128, 1)
+    ms = gemm.Measure(torch.empty((T, N), dtype=torch.float16, device="cuda"), A, X, Q, N, T, K, 128)
+    tiles = max(m.id for m in ms if m.kind == 1)
+    blocks = [m for m in ms if m.kind == 0 and m.id > tiles]
+    assert sorted((m.tile_n, m.slices) for m in blocks) == [(n, z) for n in (16, 32, 48, 64) for z in (8, 16, 32)]
+    assert all(m.grid == -(-N // m.tile_n) * m.slices // 8 for m in blocks if m.feasible)
