@@ -21,15 +21,11 @@
 //
 // A grid that leaves CUs idle splits K across workgroups as well: partial tiles through the workspace, the last
 // workgroup to arrive adds them in split order.
-#include "strip_body.h"
+#include "pipeline.h"
 
 namespace w4a16 {
 
 namespace {
-
-using strip::lds_addr;
-using strip::lds_read128;
-using strip::static_for;
 
 constexpr int kWaves = 8;
 
@@ -341,10 +337,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             }
             else {
                 uint64_t* o = reinterpret_cast<uint64_t*>(mine + ((int64_t)split * (R * H) + r0 * H + t) * 256);
-                __hip_atomic_store(o, (uint64_t)__builtin_bit_cast(uint32_t, (float)v[0]) | ((uint64_t)__builtin_bit_cast(uint32_t, (float)v[1]) << 32),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(o + 1, (uint64_t)__builtin_bit_cast(uint32_t, (float)v[2]) | ((uint64_t)__builtin_bit_cast(uint32_t, (float)v[3]) << 32),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(o, pack2(v[0], v[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(o + 1, pack2(v[2], v[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
     }
@@ -373,10 +367,10 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
             for (int u = 0; u < 4; ++u)
                 if (s0 + u < p.splits) {
-                    sum[0] += __builtin_bit_cast(float, (uint32_t)v[u][0]);
-                    sum[1] += __builtin_bit_cast(float, (uint32_t)(v[u][0] >> 32));
-                    sum[2] += __builtin_bit_cast(float, (uint32_t)v[u][1]);
-                    sum[3] += __builtin_bit_cast(float, (uint32_t)(v[u][1] >> 32));
+                    sum[0] += lo_float(v[u][0]);
+                    sum[1] += hi_float(v[u][0]);
+                    sum[2] += lo_float(v[u][1]);
+                    sum[3] += hi_float(v[u][1]);
                 }
         }
         emit(t / H, t % H, sum);

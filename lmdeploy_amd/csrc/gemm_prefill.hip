@@ -20,10 +20,7 @@
 // part: an MFMA occupies the pipe for 16 cycles and issues in 4; two vector instructions fit
 // behind each one for free, a third does not).  The MFMAs are inline assembly with the
 // accumulators tied in place in AGPRs; loads are inline assembly waited for by count.
-#include "w4a16_common.h"
-#include "w4a16_internal.h"
-
-#include <type_traits>
+#include "pipeline.h"
 
 namespace w4a16 {
 
@@ -35,38 +32,6 @@ namespace {
 // the direct global-to-LDS loads (64 lanes x 16 contiguous bytes) could not produce.
 constexpr int kRowBytes = kGroup * 2;
 
-// Compile-time loop: f(std::integral_constant<int, 0>{}), ..., f(<N-1>); gives inline assembly
-// its immediate operands.
-template<int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
-// Loads of the software pipeline.  They are issued from inline assembly, in place ("+v"), with
-// a scalar base and a per-thread 32-bit offset, and waited for by count: the compiler would
-// drain every load in flight at the loop header, exposing the memory latency once per K step.
-template<int OFF>
-__device__ __forceinline__ void gload128(u32x4_t& dst, uint32_t voff, const void* sbase)
-{
-    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "+v"(dst) : "v"(voff), "s"(sbase), "n"(OFF));
-}
-template<int OFF>
-__device__ __forceinline__ void gload32(uint32_t& dst, uint32_t voff, const void* sbase)
-{
-    asm volatile("global_load_dword %0, %1, %2 offset:%3" : "+v"(dst) : "v"(voff), "s"(sbase), "n"(OFF));
-}
-// Global memory straight into LDS: lane l's 16 bytes land at lds_base + 16 l.  The LDS base travels
-// in M0; written here (rather than through the builtin) so that the address is a scalar base
-// plus a 32-bit lane offset instead of a 64-bit lane address, which costs a register pair and an
-// add per request.
-__device__ __forceinline__ uint32_t lds_addr(const void* p)
-{
-    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)(p);
-}
 __device__ __forceinline__ void gload_lds128(uint32_t lds_base, uint32_t voff, const void* sbase)
 {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
@@ -74,38 +39,12 @@ __device__ __forceinline__ void gload_lds128(uint32_t lds_base, uint32_t voff, c
                  : "v"(voff), "s"(sbase), "s"(lds_base)
                  : "memory", "m0");
 }
-// wait until at most N of this wave's loads are in flight; tied to `v` so that no use of it can
-// be scheduled above the wait
-template<int N, typename V>
-__device__ __forceinline__ void wait_vm(V& v)
-{
-    asm volatile("s_waitcnt vmcnt(%1)" : "+v"(v) : "n"(N));
-}
-
-// LDS fragment read from inline assembly (byte address + immediate), and its wait.  Left to the
-// compiler, each activation fragment was read right before the MFMAs that use it, which then
-// waited a full LDS latency; and any compiler-visible LDS read after a direct-to-LDS load would
-// be preceded by a wait for ALL loads in flight.  Here the fragments of a sub-step are requested
-// during the previous one.
-template<int OFF>
-__device__ __forceinline__ void lds_read128(half8_t& dst, uint32_t addr)
-{
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
-}
 __device__ __forceinline__ void wait_lgkm0(half8_t& a, half8_t& b, half8_t& c, half8_t& d)
 {
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
 }
 
-__device__ __forceinline__ uint64_t pack2(float a, float b)
-{
-    return (uint64_t)__builtin_bit_cast(uint32_t, a) | ((uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
-}
-__device__ __forceinline__ float lo_float(uint64_t v) { return __builtin_bit_cast(float, (uint32_t)v); }
-__device__ __forceinline__ float hi_float(uint64_t v) { return __builtin_bit_cast(float, (uint32_t)(v >> 32)); }
-
-// Register budget: one wave per SIMD (512 registers) for the 128-register accumulator tiles,
-// two waves otherwise.  Stating it keeps the allocator from squeezing the kernel into fewer
+// Register budget: two waves per SIMD.  Stating it keeps the allocator from squeezing the kernel into fewer
 // VGPRs and parking values in AGPRs, which is fatal here: a register parked while an
 // inline-assembly load into it is still in flight is handed to another value, and the load then
 // lands on that value (the build rejects kernels that use AGPRs beyond their accumulators).
@@ -118,9 +57,7 @@ __device__ __forceinline__ float hi_float(uint64_t v) { return __builtin_bit_cas
 // has only 4 * NTW MFMAs per k32 chunk, too few to cover the LDS latency; two chunks per sub-step
 // double the cover at the price of a second set of fragment registers.
 template<int TTILES, int NTW, int WAVES, int D, int KS, int EPI>
-__global__ void __launch_bounds__(64 * WAVES)
-    __attribute__((amdgpu_waves_per_eu(TTILES * NTW * KS >= 16 && WAVES == 4 && (TTILES * NTW >= 32 || KS == 2) ? 1 : 2,
-                                       TTILES * NTW * KS >= 16 && WAVES == 4 && (TTILES * NTW >= 32 || KS == 2) ? 1 : 2)))
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
 prefill_kernel(uint16_t* __restrict__ C, const u32x4_t* __restrict__ A, const uint16_t* __restrict__ X,
                const uint32_t* __restrict__ Q, const uint16_t* R_, int N, int T, int K, int tiles_t, int tiles_n,
                float* ws, int* cnt, int epoch)

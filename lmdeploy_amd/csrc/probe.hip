@@ -10,10 +10,9 @@
 // parameters, for sweeping what the memory system gives at best.
 // probe_mfma_kernel: nothing but v_mfma_f32_16x16x32_f16 on registers, for the rate the matrix pipes reach at
 // the clock the chip settles at under them.
-#include "w4a16_common.h"
+#include "pipeline.h"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace w4a16 {
 
@@ -33,15 +32,6 @@ __global__ void __launch_bounds__(512) probe_read_kernel(const u32x4_t* __restri
     }
     const uint32_t x = acc[0] ^ acc[1] ^ acc[2] ^ acc[3];
     if (x == 0x9e3779b9u) sink[blockIdx.x] = x;  // (keeps the loads alive; practically never taken)
-}
-
-template<int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
 }
 
 // One 16-byte load per lane at sbase + voff, in place; with flag 0 it is issued under EXEC = 0: it

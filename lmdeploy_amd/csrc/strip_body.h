@@ -11,10 +11,7 @@
 // partial strips are added in LDS in slice order.
 #pragma once
 
-#include "w4a16_common.h"
-#include "w4a16_internal.h"
-
-#include <type_traits>
+#include "pipeline.h"
 
 namespace w4a16 {
 
@@ -88,12 +85,6 @@ __device__ __forceinline__ void mload128_agent(u32x4_t& dst, uint32_t voff, cons
                  : "scc");
 }
 
-// Global memory straight into LDS (no registers): lane l's 16 bytes land at lds_base + 16 l.  The LDS
-// base travels in M0.  Counts in vmcnt like any other load, and is complete there when the data is in LDS.
-__device__ __forceinline__ uint32_t lds_addr(const void* p)
-{
-    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)(p);
-}
 __device__ __forceinline__ void mload128_lds(uint32_t lds_base, uint32_t voff, const void* sbase, int flag)
 {
     uint64_t sv;
@@ -102,23 +93,6 @@ __device__ __forceinline__ void mload128_lds(uint32_t lds_base, uint32_t voff, c
                  : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(flag), [lb] "s"(lds_base)
                  : "scc", "m0", "memory");
 }
-// LDS fragment read from inline assembly: the compiler would put a wait for every load in flight in front of
-// an LDS read of its own that follows a direct-to-LDS load.
-template<int OFF>
-__device__ __forceinline__ void lds_read128(half8_t& dst, uint32_t addr)
-{
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
-}
-
-template<int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
 // Everything one wave holds for one group: R weight tiles, their Q words, and the activations of
 // the group (NX loads of four token rows x 256 bytes each, one 16-byte chunk per lane).
 // (With 2 or 4 quantisation groups per weight tile, tile r's words are spread over the lanes of q[r]: spread_q.)

@@ -18,48 +18,14 @@
 // in AGPRs; loads are inline assembly waited for by count.
 #pragma once
 
-#include "w4a16_common.h"
-#include "w4a16_internal.h"
-
-#include <type_traits>
+#include "pipeline.h"
 
 namespace w4a16 {
 
 namespace {
 
-// Compile-time loop: f(std::integral_constant<int, 0>{}), ..., f(<N-1>); gives inline assembly
-// its immediate operands.
-template<int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
-// Loads of the software pipeline.  They are issued from inline assembly, in place ("+v"), with
-// a scalar base and a per-thread 32-bit offset, and waited for by count: the compiler would
-// drain every load in flight at the loop header, exposing the memory latency once per K step.
-template<int OFF>
-__device__ __forceinline__ void gload128(u32x4_t& dst, uint32_t voff, const void* sbase)
-{
-    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "+v"(dst) : "v"(voff), "s"(sbase), "n"(OFF));
-}
-template<int OFF>
-__device__ __forceinline__ void gload32(uint32_t& dst, uint32_t voff, const void* sbase)
-{
-    asm volatile("global_load_dword %0, %1, %2 offset:%3" : "+v"(dst) : "v"(voff), "s"(sbase), "n"(OFF));
-}
-// Global memory straight into LDS: lane l's 16 bytes land at lds_base + 16 l.  The LDS base travels
-// in M0; written here (rather than through the builtin) so that the address is a scalar base
-// plus a 32-bit lane offset instead of a 64-bit lane address, which costs a register pair and an
-// add per request.  One value serves several requests, each a statement of its own: the build's assembly check
-// verifies that nothing else writes M0 in a kernel that relies on this.
-__device__ __forceinline__ uint32_t lds_addr(const void* p)
-{
-    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)(p);
-}
+// Direct-to-LDS loads whose address in LDS (M0) serves several requests, each a statement of its own: the build's assembly
+// check verifies that nothing else writes M0 in a kernel that relies on this.
 __device__ __forceinline__ void set_m0(uint32_t v)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(v) : "memory", "m0");
@@ -68,24 +34,6 @@ template<int OFF>
 __device__ __forceinline__ void gload_lds128_m0(uint32_t voff, const void* sbase)
 {
     asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
-}
-// wait until at most N of this wave's loads are in flight; tied to `v` so that no use of it can
-// be scheduled above the wait
-template<int N, typename V>
-__device__ __forceinline__ void wait_vm(V& v)
-{
-    asm volatile("s_waitcnt vmcnt(%1)" : "+v"(v) : "n"(N));
-}
-
-// LDS fragment read from inline assembly (byte address + immediate), and its wait.  Left to the
-// compiler, each activation fragment was read right before the MFMAs that use it, which then
-// waited a full LDS latency; and any compiler-visible LDS read after a direct-to-LDS load would
-// be preceded by a wait for ALL loads in flight.  Here the fragments of a sub-step are requested
-// during the previous one.
-template<int OFF>
-__device__ __forceinline__ void lds_read128(half8_t& dst, uint32_t addr)
-{
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
 // g / (1 + exp(-g)) with the quotient rounded as a division rounds it: the approximate quotient and one correction by its exact
 // remainder (Markstein), special cases by the instruction that ends the compiler's division too.  Without the scaling that
@@ -98,12 +46,6 @@ __device__ __forceinline__ float silu_quotient(float g)
     const float d = 1.f + __expf(-g), r = __builtin_amdgcn_rcpf(d), q = g * r;
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, g), r, q), d, g);
 }
-__device__ __forceinline__ uint64_t pack2(float a, float b)
-{
-    return (uint64_t)__builtin_bit_cast(uint32_t, a) | ((uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
-}
-__device__ __forceinline__ float lo_float(uint64_t v) { return __builtin_bit_cast(float, (uint32_t)v); }
-__device__ __forceinline__ float hi_float(uint64_t v) { return __builtin_bit_cast(float, (uint32_t)(v >> 32)); }
 
 // A wave computes 16 TTILES tokens x 16 NTW features in blocks of 32 x 32 (v_mfma_f32_32x32x16_f16); the four waves of a
 // workgroup are side by side along the features.  D = groups in flight per wave (2 or 4): the loads of group g + D are issued while group g is being
@@ -127,7 +69,7 @@ tile_kernel(uint16_t* __restrict__ C, const u32x4_t* __restrict__ A, const uint1
             const uint32_t* __restrict__ Q, const uint16_t* R_, int N, int T, int K, int tiles_t, int tiles_n, int epi,
             float* ws, int* cnt, int epoch)
 {
-    extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [D][TT][kRowBytes]
+    extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [D][4 TTILES][kBlock]
     constexpr int WAVES = 4;
     constexpr int TT    = 16 * TTILES;
     constexpr int kBlock = 1024 + 16, kStage = 4 * TTILES * kBlock;  // bytes of LDS
@@ -572,7 +514,7 @@ hipError_t launch_tile_one(int splits, const GemmArgs& a, const Scratch& sc, hip
                          a.R, a.N, a.T, a.K, tiles_t, tiles_n, a.epilogue, sc.ws, sc.cnt, sc.epoch);
 }
 
-// The tiles that exist (w4a16_internal.h: tile_exists), stages by what LDS holds.
+// The tiles that exist (api.cpp has their prices), stages by what LDS holds.
 template<int NQ>
 hipError_t launch_tile(const TileConfig& cf, const GemmArgs& a, const Scratch& sc, hipStream_t st)
 {
