@@ -28,8 +28,8 @@ struct Metric {
     int                id;
     bool               feasible;
     bool               prefer;
-    std::array<int, 3> cta_shape;  // {features, tokens, K slices per workgroup}
-    int                kind;       // 0 decode kernel (column blocks), 1 MFMA prefill kernel, 2 decode kernel (strips)
+    std::array<int, 3> cta_shape;  // {features, tokens, slices of w4a16_metric}
+    int                kind;       // 0 decode kernel (column blocks), 1 MFMA tiles, 2 decode kernel (strips), 3 batch kernel
     float              grid_size;
     int                best;
     float              time;       // milliseconds for `count` launches

@@ -10,10 +10,11 @@
 //   have changed, and they are not costs of anything today (those are in api.cpp).
 // * Sizes that moved from tiles to the batch kernel since (moved_to_fp32).  Bounds on size, inside which it was given
 //   everything; with 16 groups of K and more it is also the faster one there (us, batch kernel against the best tile, cold
-//   weights: 8192 x 16384 at 80 tokens 30.4 against 42.1, 4096 x 4096 at 244 13.6 against 17.1, 8192 x 1024 at 976 27.1
-//   against 27.4, 14336 x 2048 at 488 37.8 against 41.2).  With fewer groups, and where N is an odd multiple of 64, the
-//   precision costs time: 1536 x 16384 at 160 20.2 against 16.1, 512 x 8192 at 600 26.3 against 11.1, 4096 x 11200 at 384 59.8
-//   against 44.1, 4096 x 22080 at 2048 575 against 322.
+//   weights: 8192 x 16384 at 80 tokens 31.8 against 43.2, 4096 x 4096 at 244 13.2 against 17.6, 8192 x 1024 at 976 27.2
+//   against 27.4, 14336 x 2048 at 488 37.5 against 42.8).  With fewer groups, and where N is an odd multiple of 64, the
+//   precision costs time: 1536 x 16384 at 160 20.2 against 16.6, 512 x 8192 at 600 26.1 against 9.7, 4096 x 11200 at 384 57.0
+//   against 43.4, 4096 x 22080 at 2048 574 against 308.  So it does in the first set (4096 x 10944 at 3329 509 against 295,
+//   1664 x 9920 at 641 58 against 28).  No matrix of the 7B and 70B layers is that wide.
 #include "w4a16_internal.h"
 
 #include <cmath>

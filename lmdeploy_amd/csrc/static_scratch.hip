@@ -71,8 +71,9 @@ hipError_t static_scratch(Scratch* out)
 // Before a launch that counts arrivals in `sc`, of static_scratch, with `n` counters.  A launch made at once has a tag that no
 // earlier one used, and starts from whatever is there.  The replays of a recorded launch all carry one tag, and a count that
 // overlapping calls left under it would be taken for the replay's own, each time: there the counters are cleared first, by a
-// kernel (not hipMemsetAsync, whose nodes a graph may replay wrongly), and counted without a tag.  One more kernel per
-// recorded launch, 1.6 us; for launches made at once the clearing kernel cost 8192 x 1024 at 16 tokens 12.1 us against 8.0.
+// kernel (not hipMemsetAsync, whose nodes a graph may replay wrongly), and counted without a tag.  8192 x 1024 at 16 tokens, K
+// split in four: in a graph 9.1 us a launch with tags, 7.9 with the clearing kernel and without; made at once 8.0 with tags, 8.4
+// with the clearing kernel, which is a second call for the host to make.
 hipError_t prepare_static_counters(Scratch* sc, int n, hipStream_t st)
 {
     // (the null stream cannot be captured, and must not be asked while another one is)
