@@ -21,7 +21,7 @@ SOURCES = ["api.cpp", "rounding_domain.cpp", "repack.hip", "static_scratch.hip",
 
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 instructions for this target.
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
-             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=14"]
 
 
 def _hipcc() -> str:

@@ -38,12 +38,13 @@ using namespace strip;
 // RMAX = width of the wide strips (base + 1 when the column tiles do not divide evenly).
 // D = groups in flight per wave (2, or 1 for wide strips: see strip_launch).
 template<int RMAX, int TP, int EPI, int D = 2>
-__global__ void __launch_bounds__(64 * kWaves) strip_kernel(const StripParams p)
+__global__ void __launch_bounds__(64 * kWaves) strip_kernel(STRIP_ARGS)
 {
     extern __shared__ __attribute__((aligned(16))) u32x4_t smem[];  // activation patches [8][1 or 2][TP][16], then sums [8][R][H][64]
-    clock_record_start(p.clk, blockIdx.x == gridDim.x / 2 && blockIdx.y == 0 && threadIdx.x == 0);
+    const StripParams p = strip_params(STRIP_ARG_NAMES);
+    if (how & kHowClock) clock_record_start(strip_clock(), blockIdx.x == gridDim.x / 2 && blockIdx.y == 0 && threadIdx.x == 0);
     for (int pass = 0; pass < p.passes; ++pass) {
-        const int  bx   = pass * gridDim.x + blockIdx.x;
+        const int  bx   = pass * p.grid + blockIdx.x;
         const bool wide = bx < p.rem;
         const int  col0 = bx * p.base + min(bx, p.rem);
         if (pass) __syncthreads();  // the sums of the previous strip have been read out of LDS
@@ -56,7 +57,7 @@ __global__ void __launch_bounds__(64 * kWaves) strip_kernel(const StripParams p)
         }
         if (!done) strip_body<RMAX, TP, EPI, false, kWaves, NoWait, 1, D>(p, col0, smem);
     }
-    clock_record_stop(p.clk, blockIdx.x == gridDim.x / 2 && blockIdx.y == 0 && threadIdx.x == 0);
+    if (how & kHowClock) clock_record_stop(strip_clock(), blockIdx.x == gridDim.x / 2 && blockIdx.y == 0 && threadIdx.x == 0);
 }
 
 // One-tile strips at up to eight tokens: sixteen waves instead of eight, so that a wave walks half as many groups
@@ -65,12 +66,13 @@ __global__ void __launch_bounds__(64 * kWaves) strip_kernel(const StripParams p)
 // group in flight instead of two (down at eight tokens 9.7 -> 9.1 us, o 5.0 -> 4.85); at sixteen tokens, and for
 // two-tile strips, eight waves are ahead.
 template<int TP, int EPI, int D>
-__global__ void __launch_bounds__(64 * kWavesNarrow) strip_kernel_narrow(const StripParams p)
+__global__ void __launch_bounds__(64 * kWavesNarrow) strip_kernel_narrow(STRIP_ARGS)
 {
     extern __shared__ __attribute__((aligned(16))) u32x4_t smem[];
-    clock_record_start(p.clk, blockIdx.x == gridDim.x / 2 && threadIdx.x == 0);
+    const StripParams p = strip_params(STRIP_ARG_NAMES);
+    if (how & kHowClock) clock_record_start(strip_clock(), blockIdx.x == gridDim.x / 2 && threadIdx.x == 0);
     strip_body<1, TP, EPI, false, kWavesNarrow, NoWait, 1, D>(p, (int)blockIdx.x, smem);
-    clock_record_stop(p.clk, blockIdx.x == gridDim.x / 2 && threadIdx.x == 0);
+    if (how & kHowClock) clock_record_stop(strip_clock(), blockIdx.x == gridDim.x / 2 && threadIdx.x == 0);
 }
 
 template<int TP, int D>
@@ -79,9 +81,9 @@ hipError_t launch_narrow(const StripParams& p, dim3 grid, int epilogue, hipStrea
     const dim3   block(64 * kWavesNarrow);
     const size_t lds = (size_t)kWavesNarrow * std::max(1024, TP * 256);
     switch (epilogue) {
-        case kEpiGemm: return launch_kernel(strip_kernel_narrow<TP, kEpiGemm, D>, grid, block, lds, st, p);
-        case kEpiSilu: return launch_kernel(strip_kernel_narrow<TP, kEpiSilu, D>, grid, block, lds, st, p);
-        default: return launch_kernel(strip_kernel_narrow<TP, kEpiAdd, D>, grid, block, lds, st, p);
+        case kEpiGemm: return launch_strip(strip_kernel_narrow<TP, kEpiGemm, D>, grid, block, lds, st, p);
+        case kEpiSilu: return launch_strip(strip_kernel_narrow<TP, kEpiSilu, D>, grid, block, lds, st, p);
+        default: return launch_strip(strip_kernel_narrow<TP, kEpiAdd, D>, grid, block, lds, st, p);
     }
 }
 
@@ -98,7 +100,7 @@ hipError_t launch_rt(const StripParams& p, dim3 grid, size_t lds, int epilogue, 
             const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kfn), 8 * kMaxR32 * 2 * 1024, raised);  \
             if (e != hipSuccess) return e;                                                                             \
         }                                                                                                              \
-        return launch_kernel(kfn, grid, block, lds, st, p);                                                            \
+        return launch_strip(kfn, grid, block, lds, st, p);                                                             \
     } while (0)
     switch (epilogue) {
         case kEpiGemm: W4A16_LAUNCH(kEpiGemm);
@@ -201,7 +203,7 @@ hipError_t strip_launch(int cus, int per_cu, int block_t, const GemmArgs& a, hip
     const int   tp = block_t == 32 ? 32 : (a.T <= 4 ? 4 : (a.T <= 8 ? 8 : 16));
     const int   h  = tp > 16 ? tp / 16 : 1;
     StripParams p{a.C, reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.R, a.N, a.T, a.K, pl.base, pl.rem,
-                  a.epilogue, pl.passes, a.clk};
+                  a.epilogue, pl.passes, pl.strips, a.clk};
     const dim3   grid(pl.strips, (a.T + block_t - 1) / block_t);
     // per wave: the sums of its strip, over its activation patch(es) - two for 32 tokens, which arrive straight from memory
     const size_t lds = (size_t)kWaves * std::max(pl.rmax * h * 1024, tp * 256 * (tp >= kDmaTokens ? 2 : 1));

@@ -12,11 +12,12 @@ namespace {
 using namespace strip;
 
 template<int RMAX, int TP, int D, int NQ>
-__global__ void __launch_bounds__(64 * kWaves) strip_kernel_q(const StripParams p)
+__global__ void __launch_bounds__(64 * kWaves) strip_kernel_q(STRIP_ARGS)
 {
     extern __shared__ __attribute__((aligned(16))) u32x4_t smem[];
+    const StripParams p = strip_params(STRIP_ARG_NAMES);
     for (int pass = 0; pass < p.passes; ++pass) {
-        const int  bx   = pass * gridDim.x + blockIdx.x;
+        const int  bx   = pass * p.grid + blockIdx.x;
         const bool wide = bx < p.rem;
         const int  col0 = bx * p.base + min(bx, p.rem);
         if (pass) __syncthreads();  // the sums of the previous strip have been read out of LDS
@@ -32,9 +33,10 @@ __global__ void __launch_bounds__(64 * kWaves) strip_kernel_q(const StripParams 
 }
 
 template<int TP, int D, int NQ>
-__global__ void __launch_bounds__(64 * kWavesNarrow) strip_kernel_q_narrow(const StripParams p)
+__global__ void __launch_bounds__(64 * kWavesNarrow) strip_kernel_q_narrow(STRIP_ARGS)
 {
     extern __shared__ __attribute__((aligned(16))) u32x4_t smem[];
+    const StripParams p = strip_params(STRIP_ARG_NAMES);
     strip_body<1, TP, kEpiRuntime, false, kWavesNarrow, NoWait, NQ, D>(p, (int)blockIdx.x, smem);
 }
 
@@ -42,9 +44,9 @@ template<int RMAX, int D, int NQ>
 hipError_t launch_tp(int tp, const StripParams& p, dim3 grid, size_t lds, hipStream_t st)
 {
     const dim3 block(64 * kWaves);
-    if (tp == 4) return launch_kernel(strip_kernel_q<RMAX, 4, D, NQ>, grid, block, lds, st, p);
-    if (tp == 8) return launch_kernel(strip_kernel_q<RMAX, 8, D, NQ>, grid, block, lds, st, p);
-    return launch_kernel(strip_kernel_q<RMAX, 16, D, NQ>, grid, block, lds, st, p);
+    if (tp == 4) return launch_strip(strip_kernel_q<RMAX, 4, D, NQ>, grid, block, lds, st, p);
+    if (tp == 8) return launch_strip(strip_kernel_q<RMAX, 8, D, NQ>, grid, block, lds, st, p);
+    return launch_strip(strip_kernel_q<RMAX, 16, D, NQ>, grid, block, lds, st, p);
 }
 
 template<int NQ>
@@ -53,8 +55,8 @@ hipError_t launch_q(const StripPlan& pl, int tp, const StripParams& p, dim3 grid
     if (pl.narrow) {
         const dim3   block(64 * kWavesNarrow);
         const size_t lds = (size_t)kWavesNarrow * std::max(1024, tp * 256);
-        if (tp == 4) return launch_kernel(strip_kernel_q_narrow<4, 2, NQ>, grid, block, lds, st, p);
-        return launch_kernel(strip_kernel_q_narrow<8, 1, NQ>, grid, block, lds, st, p);
+        if (tp == 4) return launch_strip(strip_kernel_q_narrow<4, 2, NQ>, grid, block, lds, st, p);
+        return launch_strip(strip_kernel_q_narrow<8, 1, NQ>, grid, block, lds, st, p);
     }
     const size_t lds = (size_t)kWaves * std::max(pl.rmax * 1024, tp * 256);
     switch (pl.rmax) {
@@ -77,7 +79,7 @@ hipError_t strip_groups_launch(int nq, int cus, int per_cu, const GemmArgs& a, h
     if (!pl.ok || (nq != 2 && nq != 4)) return hipErrorInvalidValue;
     const int   tp = a.T <= 4 ? 4 : (a.T <= 8 ? 8 : 16);
     StripParams p{a.C, reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.R, a.N, a.T, a.K, pl.base, pl.rem,
-                  a.epilogue, pl.passes};
+                  a.epilogue, pl.passes, pl.strips};
     const dim3  grid(pl.strips, (a.T + 15) / 16);
     return nq == 2 ? launch_q<2>(pl, tp, p, grid, st) : launch_q<4>(pl, tp, p, grid, st);
 }

@@ -34,64 +34,106 @@ struct StripParams {
     int             rem;   // the first `rem` strips have base + 1
     int             epilogue;  // read by kernels whose epilogue is chosen at run time (EPI == kEpiRuntime)
     int             passes;    // strips per workgroup, one after the other (strip number = pass * workgroups + workgroup)
-    unsigned long long* clk = nullptr;  // measurement aid (clock_record_start / _stop); null in every ordinary launch
+    int             grid = 0;  // workgroups side by side
+    unsigned long long* clk = nullptr;  // measurement aid (clock_record_start / _stop); null in every ordinary launch (host side)
 };
+
+// The kernels take these one by one: the first fourteen words of a kernel's arguments are put into scalar registers by the
+// command processor (kernarg preloading, which does not look into a struct), so that the first loads go out at once instead of
+// behind two trips to memory for the pointers.  What only the epilogue needs comes last.  A narrow matrix is done a few
+// microseconds after its launch, and everything in front of the first load counts in full: with this, addresses that advance
+// instead of being multiplied out for every group, and one change of the mask for up to four loads, 4096 x 4096 at one token
+// went from 4.43 to 4.10 us, 4096 x 12288 7.33 -> 6.95, 4096 x 22016 11.42 -> 10.95, 11008 x 4096 7.05 -> 6.62 (cold weights).
+#define STRIP_ARGS                                                                                                     \
+    const u32x4_t *A, const uint16_t *X, const uint32_t *Q, int N, int T, int K, int rem, int passes, uint32_t how,    \
+        uint16_t *C, const uint16_t *Rsd, unsigned long long *clk
+#define STRIP_ARG_NAMES A, X, Q, N, T, K, rem, passes, how, C, Rsd, clk
+// `how`: workgroups side by side (16 bits, read where they take several strips: one for each CU then), width of a narrow strip (8), epilogue (2), and whether the clock is recorded
+constexpr uint32_t kHowClock = 1u << 31;
+__device__ __forceinline__ StripParams strip_params(STRIP_ARGS)
+{
+    return StripParams{C, A, X, Q, Rsd, N, T, K, (int)(how >> 16 & 0xff), rem, (int)(how >> 28 & 3), passes, (int)(how & 0xffff)};
+}
+template<typename F>
+hipError_t launch_strip(F* kernel, dim3 grid, dim3 block, size_t lds, hipStream_t st, const StripParams& p)
+{
+    const uint32_t how = ((uint32_t)p.grid & 0xffff) | (uint32_t)p.base << 16 | (uint32_t)p.epilogue << 28 | (p.clk ? kHowClock : 0);
+    return launch_kernel(kernel, grid, block, lds, st, p.A, p.X, p.Q, p.N, p.T, p.K, p.rem, p.passes, how, p.C, p.Rsd, p.clk);
+}
+// The measurement aid's pointer is read where it is used, and not, as the compiler would have it, up front with a wait for it.
+__device__ __forceinline__ unsigned long long* strip_clock()
+{
+    typedef __attribute__((address_space(1))) unsigned long long* counters;
+    auto args = (__attribute__((address_space(4))) const char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return (unsigned long long*)*(__attribute__((address_space(4))) const counters*)(args + 64);
+}
 
 constexpr int kEpiRuntime = 3;  // template value: take the epilogue from StripParams
 
 // Loads of the software pipeline: issued from inline assembly, in place ("+v"), with a scalar
 // base, a per-lane 32-bit offset and an immediate, and waited for by count (the compiler would
-// drain every load in flight at the loop header).  `LOADS(...)` wraps a few of them in an EXEC
-// mask: with flag 0 the instructions still issue and still count in vmcnt, but touch neither
-// memory nor their destination, which lets the last trips of a loop skip their refills without
-// a branch - the number of loads in flight stays a compile-time constant.
-#define W4A16_MASKED(body)                                                                                             \
-    "s_mov_b64 %[sv], exec\n\ts_cmp_lg_u32 %[mk], 0\n\ts_cselect_b64 exec, exec, 0\n\t" body "s_mov_b64 exec, %[sv]"
+// drain every load in flight at the loop header).  They run under an EXEC mask of all lanes or none
+// (every lane is active around them): with none the instructions still issue and still count in vmcnt, but touch
+// neither memory nor their destination, which lets the last trips of a loop skip their refills without
+// a branch - the number of loads in flight stays a compile-time constant.  Up to four loads share one change of the mask:
+// the scalar instructions between the loads of all waves of a SIMD add up.
+#define W4A16_MASKED(body) "s_mov_b64 exec, %[mk]\n\t" body "s_mov_b64 exec, -1"
+#define W4A16_LOAD(INS, i, CACHE) INS " %[d" #i "], %[vo], %[sb] offset:%[i" #i "]" CACHE "\n\t"
+#define W4A16_LOADS(INS, CACHE, N, OFF)                                                                                \
+    if constexpr (N == 1)                                                                                              \
+        asm volatile(W4A16_MASKED(W4A16_LOAD(INS, 0, CACHE))                                                           \
+                     : [d0] "+v"(dst[0])                                                                               \
+                     : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(mask), [i0] "n"(OFF(0)));                             \
+    if constexpr (N == 2)                                                                                              \
+        asm volatile(W4A16_MASKED(W4A16_LOAD(INS, 0, CACHE) W4A16_LOAD(INS, 1, CACHE))                                 \
+                     : [d0] "+v"(dst[0]), [d1] "+v"(dst[1])                                                            \
+                     : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(mask), [i0] "n"(OFF(0)), [i1] "n"(OFF(1)));           \
+    if constexpr (N == 3)                                                                                              \
+        asm volatile(W4A16_MASKED(W4A16_LOAD(INS, 0, CACHE) W4A16_LOAD(INS, 1, CACHE) W4A16_LOAD(INS, 2, CACHE))       \
+                     : [d0] "+v"(dst[0]), [d1] "+v"(dst[1]), [d2] "+v"(dst[2])                                         \
+                     : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(mask), [i0] "n"(OFF(0)), [i1] "n"(OFF(1)),            \
+                       [i2] "n"(OFF(2)));                                                                              \
+    if constexpr (N == 4)                                                                                              \
+        asm volatile(W4A16_MASKED(W4A16_LOAD(INS, 0, CACHE) W4A16_LOAD(INS, 1, CACHE) W4A16_LOAD(INS, 2, CACHE)        \
+                                      W4A16_LOAD(INS, 3, CACHE))                                                       \
+                     : [d0] "+v"(dst[0]), [d1] "+v"(dst[1]), [d2] "+v"(dst[2]), [d3] "+v"(dst[3])                      \
+                     : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(mask), [i0] "n"(OFF(0)), [i1] "n"(OFF(1)),            \
+                       [i2] "n"(OFF(2)), [i3] "n"(OFF(3)));
 
-template<int IM>
-__device__ __forceinline__ void mload32(uint32_t& dst, uint32_t voff, const void* sbase, int flag)
+// N (zero, scale) words, of tiles FIRST, FIRST + 1, ... of a strip
+template<int N, int FIRST>
+__device__ __forceinline__ void mload_q(uint32_t* dst, uint32_t voff, const void* sbase, uint64_t mask)
 {
-    uint64_t sv;
-    asm volatile(W4A16_MASKED("global_load_dword %[d], %[vo], %[sb] offset:%[im]\n\t")
-                 : [d] "+v"(dst), [sv] "=&s"(sv)
-                 : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(flag), [im] "n"(IM)
-                 : "scc");
+#define W4A16_OFF(i) (FIRST + (i)) * 64
+    W4A16_LOADS("global_load_dword", "", N, W4A16_OFF)
+#undef W4A16_OFF
 }
-template<int IM>
-__device__ __forceinline__ void mload128_nt(u32x4_t& dst, uint32_t voff, const void* sbase, int flag)
+// N adjacent weight tiles
+template<int N>
+__device__ __forceinline__ void mload_w(u32x4_t* dst, uint32_t voff, const void* sbase, uint64_t mask)
 {
-    uint64_t sv;
-    asm volatile(W4A16_MASKED("global_load_dwordx4 %[d], %[vo], %[sb] offset:%[im] nt\n\t")
-                 : [d] "+v"(dst), [sv] "=&s"(sv)
-                 : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(flag), [im] "n"(IM)
-                 : "scc");
+#define W4A16_OFF(i) (i) * 1024
+    W4A16_LOADS("global_load_dwordx4", " nt", N, W4A16_OFF)
+#undef W4A16_OFF
 }
-__device__ __forceinline__ void mload128(u32x4_t& dst, uint32_t voff, const void* sbase, int flag)
+__device__ __forceinline__ void mload128(u32x4_t& dst, uint32_t voff, const void* sbase, uint64_t mask)
 {
-    uint64_t sv;
-    asm volatile(W4A16_MASKED("global_load_dwordx4 %[d], %[vo], %[sb]\n\t")
-                 : [d] "+v"(dst), [sv] "=&s"(sv)
-                 : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(flag)
-                 : "scc");
+    asm volatile(W4A16_MASKED("global_load_dwordx4 %[d], %[vo], %[sb]\n\t") : [d] "+v"(dst) : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(mask));
 }
 // the same at agent scope: for data that another workgroup of the same launch, possibly on another
 // XCD (each XCD has its own L2), has written with agent-scope stores
-__device__ __forceinline__ void mload128_agent(u32x4_t& dst, uint32_t voff, const void* sbase, int flag)
+__device__ __forceinline__ void mload128_agent(u32x4_t& dst, uint32_t voff, const void* sbase, uint64_t mask)
 {
-    uint64_t sv;
-    asm volatile(W4A16_MASKED("global_load_dwordx4 %[d], %[vo], %[sb] sc1\n\t")
-                 : [d] "+v"(dst), [sv] "=&s"(sv)
-                 : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(flag)
-                 : "scc");
+    asm volatile(W4A16_MASKED("global_load_dwordx4 %[d], %[vo], %[sb] sc1\n\t") : [d] "+v"(dst) : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(mask));
 }
 
-__device__ __forceinline__ void mload128_lds(uint32_t lds_base, uint32_t voff, const void* sbase, int flag)
+__device__ __forceinline__ void mload128_lds(uint32_t lds_base, uint32_t voff, const void* sbase, uint64_t mask)
 {
-    uint64_t sv;
     asm volatile("s_mov_b32 m0, %[lb]\n\t" W4A16_MASKED("global_load_lds_dwordx4 %[vo], %[sb]\n\t")
-                 : [sv] "=&s"(sv)
-                 : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(flag), [lb] "s"(lds_base)
-                 : "scc", "m0", "memory");
+                 :
+                 : [vo] "v"(voff), [sb] "s"(sbase), [mk] "s"(mask), [lb] "s"(lds_base)
+                 : "m0", "memory");
 }
 // Everything one wave holds for one group: R weight tiles, their Q words, and the activations of
 // the group (NX loads of four token rows x 256 bytes each, one 16-byte chunk per lane).
@@ -128,8 +170,8 @@ __device__ __forceinline__ void strip_body(const StripParams& p, int col0, u32x4
     const int c    = lane & 15;
     const int b    = lane >> 4;
     const int N = p.N, T = p.T, K = p.K;
-    const int G  = K / kGroup;
-    const int NT = N / kTileN;
+    const int G  = (int)((uint32_t)K / kGroup);
+    const int NT = (int)((uint32_t)N / kTileN);
     // H row blocks of 16 tokens share every unpacked weight (H = 2 for the 32-token variant)
     constexpr int H  = TP > 16 ? TP / 16 : 1;
     const int     t0 = SEQ ? 0 : blockIdx.y * (16 * H);
@@ -138,9 +180,7 @@ __device__ __forceinline__ void strip_body(const StripParams& p, int col0, u32x4
     // this wave's groups: wave, wave + 8, wave + 16, ...  Interleaved rather than blocked, so that
     // at any moment the whole chip reads one contiguous run of a few dozen group rows of the
     // group-major weight array instead of eight distant ones (measured: DRAM prefers that).
-    const int g0  = wave;
-    const int cnt = (G - wave + NW - 1) / NW;  // 0 if wave >= G
-    constexpr int kStep = NW;
+    const int cnt = (int)((uint32_t)(G - wave + NW - 1) / NW);  // 0 if wave >= G
     // per-lane byte offsets; everything that depends on the group is scalar
     const uint32_t w_off = (uint32_t)(lane * 16);                    // + (g * NT + col0 + r) * 1024
     const uint32_t q_off = (uint32_t)((b % NQ * N + c) * 4);         // + (g * NQ * N + (col0 + r) * 16) * 4
@@ -182,35 +222,34 @@ __device__ __forceinline__ void strip_body(const StripParams& p, int col0, u32x4
             xr_at[h][j] = r * 16 + ((4 * j + b) ^ (r & 15));
         }
 
-    const char* Ab = reinterpret_cast<const char*>(p.A) + (int64_t)col0 * 1024;
-    const char* Qb = reinterpret_cast<const char*>(p.Q) + (int64_t)col0 * 64;
-    const char* Xb = reinterpret_cast<const char*>(p.X);
+    // Where the next requests go.  The first stages are requested unmasked, by waves that have no group for them too: those
+    // ask for their last group again, or for the last group there is.
+    const uint32_t gw = (uint32_t)min(wave, G - 1);
+    const char*    wp = reinterpret_cast<const char*>(p.A) + (uint64_t)(gw * (uint32_t)NT + (uint32_t)col0) * 1024;
+    const char*    qp = reinterpret_cast<const char*>(p.Q) + ((uint64_t)(gw * NQ) * (uint32_t)N + (uint64_t)(uint32_t)col0 * kTileN) * 4;
+    const char*    xp = reinterpret_cast<const char*>(p.X) + (uint64_t)gw * 256;
+    const uint64_t w_step = (uint64_t)(uint32_t)NT * (NW * 1024), q_step = (uint64_t)(uint32_t)N * (NQ * NW * 4);
 
-    // All loads of group g into stage s (number d); enable = false turns them into no-ops that still count.
+    // All loads of the next group into stage s (number d); a mask of 0 turns them into no-ops that still count.
     using StageT = Stage<R, NXR>;
     static_assert(NQ == 1 || ((NQ == 2 || NQ == 4) && H == 1), "group sizes 128, 64 and 32");
-    auto issue_x = [&](StageT& s, int d, int g, bool enable) {
-        const int flag = __builtin_amdgcn_readfirstlane(enable ? 1 : 0);
+    auto issue_x = [&](StageT& s, int d, uint64_t mask) {
         static_for<0, NX>([&](auto i) {
-            if constexpr (XDMA) mload128_lds(xw_lds + (uint32_t)(d * TP * 256 + i * 1024), x_off[i], Xb + (int64_t)g * 256, flag);
-            else if constexpr (SEQ) mload128_agent(s.x[i], x_off[i], Xb + (int64_t)g * 256, flag);
-            else mload128(s.x[i], x_off[i], Xb + (int64_t)g * 256, flag);
+            if constexpr (XDMA) mload128_lds(xw_lds + (uint32_t)(d * TP * 256 + i * 1024), x_off[i], xp, mask);
+            else if constexpr (SEQ) mload128_agent(s.x[i], x_off[i], xp, mask);
+            else mload128(s.x[i], x_off[i], xp, mask);
         });
     };
-    auto issue_wq = [&](StageT& s, int g, bool enable) {
-        const int flag = __builtin_amdgcn_readfirstlane(enable ? 1 : 0);
-        const char* qg = Qb + (int64_t)g * NQ * N * 4;
-        static_for<0, R>([&](auto r) { mload32<r * 64>(s.q[r], q_off, qg, flag); });
-        // the tiles of a group are contiguous; immediates reach 4 KiB, so every fourth tile gets a new base
-        static_for<0, R>([&](auto r) {
-            const char* wg = Ab + ((int64_t)g * NT + (r / 4) * 4) * 1024;
-            mload128_nt<(r % 4) * 1024>(s.w[r], w_off, wg, flag);
-        });
+    auto issue_wq = [&](StageT& s, uint64_t mask) {
+        static_for<0, (R + 3) / 4>([&](auto r4) { mload_q<(R - r4 * 4 < 4 ? R - r4 * 4 : 4), r4 * 4>(s.q + r4 * 4, q_off, qp, mask); });
+        // (the tiles of a group are contiguous; immediates reach 4 KiB, so every fourth tile gets a new base)
+        static_for<0, (R + 3) / 4>([&](auto r4) { mload_w<(R - r4 * 4 < 4 ? R - r4 * 4 : 4)>(s.w + r4 * 4, w_off, wp + r4 * 4096, mask); });
     };
-    auto issue = [&](StageT& s, int d, int g, bool enable) {
-        issue_x(s, d, g, enable);
-        issue_wq(s, g, enable);
+    auto issue = [&](StageT& s, int d, uint64_t mask) {
+        issue_x(s, d, mask);
+        issue_wq(s, mask);
     };
+    constexpr uint64_t kAll = ~0ull;
     constexpr int kLoads = 2 * R + NX;  // loads per stage
 
     const UnpackConsts uc;
@@ -450,49 +489,56 @@ __device__ __forceinline__ void strip_body(const StripParams& p, int col0, u32x4
     // measured slower: the unrolled loop body grows with D and is executed only once or twice.)
     static_assert((D - 1) * kLoads <= 63, "vmcnt is a 6-bit counter");
     StageT st[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) st[d].w[r] = u32x4_t{0, 0, 0, 0};
-#pragma unroll
-        for (int r = 0; r < R; ++r) st[d].q[r] = 0;
-#pragma unroll
-        for (int i = 0; i < NXR; ++i) st[d].x[i] = u32x4_t{0, 0, 0, 0};
-    }
 
     // One group: wait for the stage (exactly D - 1 younger stages are in flight behind it), use
     // it, refill it.  Nothing of a stage may be live when it is refilled (the refill is in place
     // and asynchronous), so the scheduler must not move the stage's arithmetic below its refill.
-    auto step = [&](auto dc, bool use, int refill_group, bool refill) {
+    auto step = [&](auto dc, bool use, int left) {  // (a group to refill with: left < 0)
         constexpr int d = decltype(dc)::value;
         StageT&       s = st[d];
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * kLoads) : "memory");
         pin(s);
         if (use) compute(s, dc);
         __builtin_amdgcn_sched_barrier(0);
-        issue(s, d, min(refill_group, G - 1), refill);
+        wp += w_step;
+        qp += q_step;
+        xp += NW * 256;
+        issue(s, d, (uint64_t)(int64_t)__builtin_amdgcn_readfirstlane(left >> 31));
     };
 
+    const bool second = D == 2 && cnt > 1;  // a second group to advance to
     if constexpr (SEQ) {
         // weights first (they depend on nothing), then wait for the producers of the activations, then the
         // activations; all of it complete before the loop, whose counted waits assume whole stages in order
-#pragma unroll
-        for (int d = 0; d < D; ++d) issue_wq(st[d], min(g0 + d * kStep, G - 1), d < cnt);
+        issue_wq(st[0], kAll);
+        if constexpr (D == 2) {
+            wp += second ? w_step : 0;
+            qp += second ? q_step : 0;
+            issue_wq(st[1], kAll);
+        }
         inputs_ready();
-#pragma unroll
-        for (int d = 0; d < D; ++d) issue_x(st[d], d, min(g0 + d * kStep, G - 1), d < cnt);
+        issue_x(st[0], 0, kAll);
+        if constexpr (D == 2) {
+            xp += second ? NW * 256 : 0;
+            issue_x(st[1], 1, kAll);
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     else {
-#pragma unroll
-        for (int d = 0; d < D; ++d) issue(st[d], d, min(g0 + d * kStep, G - 1), d < cnt);
+        issue(st[0], 0, kAll);
+        if constexpr (D == 2) {
+            wp += second ? w_step : 0;
+            qp += second ? q_step : 0;
+            xp += second ? NW * 256 : 0;
+            issue(st[1], 1, kAll);
+        }
     }
     // D groups per trip, so that each stage keeps its registers; all conditions are wave-uniform
     // and none of them surrounds a load.
     for (int i = 0; i < cnt; i += D) {
         static_for<0, D>([&](auto dc) {
             constexpr int d = decltype(dc)::value;
-            step(dc, i + d < cnt, g0 + (i + d + D) * kStep, i + d + D < cnt);
+            step(dc, i + d < cnt, i + d + D - cnt);
         });
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the masked refills of the last trip
