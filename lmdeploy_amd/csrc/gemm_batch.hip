@@ -29,19 +29,37 @@ namespace {
 
 constexpr int kWaves = 8;
 
-struct BatchParams {
-    uint16_t*       C;
+// The kernel takes its arguments one by one: the first fourteen words are preloaded into scalar registers (see
+// strip_body.h), and they are what it takes to issue the first loads.  The place of a workgroup comes out of them without a
+// division: three of those, one of them 64 bits wide, took longer than a K step (16 tokens, us: 8192 x 1024 split in four 6.6 -> 6.1,
+// 4096 x 4096 5.7 -> 5.1, 4096 x 12288 8.7 -> 8.2; at 48 tokens 12.0 -> 11.3).
+struct BatchArgs {
     const u32x4_t*  A;
     const uint16_t* X;
     const uint32_t* Q;
-    const uint16_t* Rsd;
     int             N, T, K;
-    int             strips, tiles_t, splits;
-    int             epilogue;
+    uint32_t        strips, tiles_t;
+    uint32_t        by_strips, by_tiles_t;  // their reciprocals (divide_by)
+    uint32_t        how;                    // log2 of the K splits (8 bits), epilogue
+    uint16_t*       C;
+    const uint16_t* Rsd;
     float*          ws;
     int*            cnt;
     int             epoch;
 };
+
+// n / d for n below some bound: d == 1 has the reciprocal 0, the others floor(2^32 / d) + 1 (exact while n d < 2^32, Granlund
+// and Montgomery), or 1 where the bound does not allow that and n is divided by d.
+uint32_t reciprocal(uint64_t bound, uint32_t d)
+{
+    return d == 1 ? 0 : bound * d < (1ull << 32) ? (uint32_t)((1ull << 32) / d) + 1 : 1;
+}
+__device__ __forceinline__ uint32_t divide_by(uint32_t n, uint32_t d, uint32_t reciprocal)
+{
+    if (reciprocal == 0) return n;
+    if (reciprocal == 1) return n / d;
+    return __umulhi(n, reciprocal);
+}
 
 // Loads of the software pipeline, waited for by count.  Their outputs are not tied to the value they replace: nothing
 // reads a stage between its refill and its wait, and the register allocator then has no reason to move a value whose
@@ -89,7 +107,9 @@ __device__ __forceinline__ void wait_frags(half8_t (&x)[H])
 }
 
 template<int R, int H, int NQ>
-__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) batch_kernel(const BatchParams p)
+__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) 
+batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int T, int K, uint32_t strips, uint32_t tiles_t,
+             uint32_t by_strips, uint32_t by_tiles_t, uint32_t how, uint16_t* C, const uint16_t* Rsd, float* ws, int* counters, int epoch)
 {
     extern __shared__ __attribute__((aligned(16))) u32x4_t smem[];  // patches [8 waves][2][16 H rows][8 chunks], then sums
     constexpr int TP     = 16 * H;
@@ -102,26 +122,27 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c    = lane & 15;
     const int b    = lane >> 4;
-    const int N = p.N, T = p.T, K = p.K;
-    const int G  = K / kGroup;
-    const int NT = N / kTileN;
+    const int G  = (int)((uint32_t)K / kGroup);
+    const int NT = (int)((uint32_t)N / kTileN);
 
     // Workgroups are dealt round-robin to the 8 XCDs; each gets a contiguous run, the token tiles of a strip next to
     // each other (they share its weights), the splits of K outermost (each touches its own part of the activations).
-    const int total = gridDim.x;
-    int       id    = blockIdx.x;
+    const uint32_t log_splits = how & 0xff, splits = 1u << log_splits;
+    const uint32_t total      = (strips * tiles_t) << log_splits;
+    uint32_t       id         = blockIdx.x;
     if (total % 8 == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-    const int tile_t = id % p.tiles_t;
-    const int strip  = id / p.tiles_t % p.strips;
-    const int split  = id / (p.tiles_t * p.strips);
+    const uint32_t row    = divide_by(id, tiles_t, by_tiles_t);  // of strips, split by split
+    const int      tile_t = (int)(id - row * tiles_t);
+    const uint32_t split  = log_splits ? divide_by(row, strips, by_strips) : 0;
+    const int      strip  = (int)(row - split * strips);
     // the last strip may overlap its neighbour: it then leaves the tiles below `first` to it
     const int first = strip * R;
     const int col0  = min(first, NT - R);
     const int t0    = tile_t * TP;
-    const int gb    = (int)((int64_t)G * split / p.splits);
-    const int ge    = (int)((int64_t)G * (split + 1) / p.splits);
+    const int gb    = (int)((uint32_t)G * split >> log_splits);  // (K below 2^31: G splits in 32 bits)
+    const int ge    = (int)((uint32_t)G * (split + 1) >> log_splits);
     const int g0    = gb + wave;  // this wave's groups: every eighth
-    const int cnt   = (ge - g0 + kWaves - 1) / kWaves;
+    const int cnt   = (int)((uint32_t)(ge - g0 + kWaves - 1) / kWaves);  // (never negative: at least one group per split)
     // The loop takes them in pairs, without a branch around anything: an odd number is padded in front with a group
     // whose activations are zeros in LDS (and whose weights are those of the first real group).
     const int pad   = cnt & 1;
@@ -147,10 +168,10 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     for (int j = 0; j < 2; ++j) xr[j] = patch + (uint32_t)(c * 128 + (((4 * j + b) ^ (c & 7) ^ (c >> 3)) & 7) * 16);
 
     // where the next requests go: weights, (zero, scale) words and activations advance by eight groups at a time
-    const int64_t w_step = (int64_t)NT * (kWaves * 1024), q_step = (int64_t)NQ * N * (kWaves * 4);
-    const char*   wp = reinterpret_cast<const char*>(p.A) + ((int64_t)g0 * NT + col0) * 1024;
-    const char*   qp = reinterpret_cast<const char*>(p.Q) + ((int64_t)g0 * NQ * N + col0 * kTileN) * 4;
-    const char*   xp = reinterpret_cast<const char*>(p.X) + (uint32_t)t0 * ((uint32_t)K * 2) + (int64_t)g0 * 256 - 3072;
+    const uint64_t w_step = (uint64_t)(uint32_t)NT * (kWaves * 1024), q_step = (uint64_t)(uint32_t)N * (NQ * kWaves * 4);
+    const char*    wp = reinterpret_cast<const char*>(A) + (uint64_t)((uint32_t)g0 * (uint32_t)NT + (uint32_t)col0) * 1024;
+    const char*    qp = reinterpret_cast<const char*>(Q) + ((uint64_t)((uint32_t)g0 * NQ) * (uint32_t)N + (uint64_t)(uint32_t)col0 * kTileN) * 4;
+    const char*    xp = reinterpret_cast<const char*>(X) + ((uint32_t)t0 * ((uint32_t)K * 2) + (uint64_t)((uint32_t)g0 * 256)) - 3072;
 
     struct Stage {
         u32x4_t  w[R];
@@ -280,7 +301,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
         step(S1{}, no{}, no{});
     }
 
-    const int epi  = p.epilogue;
+    const int epi  = (int)(how >> 8);
     auto      emit = [&](int r, int h, const float4_t v) {  // lane (c, b): token t0 + 16h + c, features n .. n + 3
         const int token = t0 + 16 * h + c;
         if (token >= T || col0 + r < first) return;
@@ -291,18 +312,18 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             const half_t o0 = (half_t)(ga / (1.f + __expf(-ga)) * ua);
             const half_t o1 = (half_t)(gc / (1.f + __expf(-gc)) * uc2);
             const uint32_t o = as_u32(half2_t{o0, o1});
-            __builtin_memcpy(p.C + (int64_t)token * (N / 2) + (n >> 1), &o, 4);
+            __builtin_memcpy(C + (int64_t)token * (N / 2) + (n >> 1), &o, 4);
             return;
         }
         uint2 o{as_u32(half2_t{h0, h1}), as_u32(half2_t{h2, h3})};
         if (epi == kEpiAdd) {
             uint2 rr;
-            __builtin_memcpy(&rr, p.Rsd + (int64_t)token * N + n, 8);  // (four bytes of alignment are all that is asked for)
+            __builtin_memcpy(&rr, Rsd + (int64_t)token * N + n, 8);  // (four bytes of alignment are all that is asked for)
             const half2_t r0 = as_half2(rr.x), r1 = as_half2(rr.y);
             o.x = as_u32(half2_t{(half_t)((float)r0[0] + (float)h0), (half_t)((float)r0[1] + (float)h1)});
             o.y = as_u32(half2_t{(half_t)((float)r1[0] + (float)h2), (half_t)((float)r1[1] + (float)h3)});
         }
-        __builtin_memcpy(p.C + (int64_t)token * N + n, &o, 8);
+        __builtin_memcpy(C + (int64_t)token * N + n, &o, 8);
     };
 
     // ---- add the eight slices in LDS, in wave order, four columns of tiles at a time (they fill the patches) ----
@@ -315,8 +336,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     constexpr int RC   = R < 4 ? R : 4;
     float4_t*     red4 = reinterpret_cast<float4_t*>(smem);
     const float*  red  = reinterpret_cast<const float*>(smem);
-    const int     tile = strip * p.tiles_t + tile_t;
-    float* const  mine = p.ws + ((int64_t)tile * p.splits) * (R * H) * 256 + lane * 4;
+    const int     tile = (int)(strip * tiles_t + tile_t);
+    float* const  mine = ws + ((int64_t)tile * (int)splits) * (R * H) * 256 + lane * 4;
 #pragma unroll
     for (int r0 = 0; r0 < R; r0 += RC) {
         __syncthreads();
@@ -332,41 +353,41 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             for (int s = 0; s < kWaves; ++s)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[i] += red[(s * RC * H + t) * 256 + get_at[i]];
-            if (p.splits == 1) {
+            if ((int)splits == 1) {
                 emit(r0 + t / H, t % H, v);
             }
             else {
-                uint64_t* o = reinterpret_cast<uint64_t*>(mine + ((int64_t)split * (R * H) + r0 * H + t) * 256);
+                uint64_t* o = reinterpret_cast<uint64_t*>(mine + ((int64_t)(int)split * (R * H) + r0 * H + t) * 256);
                 __hip_atomic_store(o, pack2(v[0], v[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(o + 1, pack2(v[2], v[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
     }
-    if (p.splits == 1) return;
+    if ((int)splits == 1) return;
 
     // ---- split K: as in the tile kernels, stores through to memory, an arrival counter, the last one adds ----
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     int* const last_flag = reinterpret_cast<int*>(smem);
     if (tid == 0) {
-        const bool last = arrive_last(p.cnt + tile, p.splits, p.epoch);
+        const bool last = arrive_last(counters + tile, (int)splits, epoch);
         *last_flag = last;
     }
     __syncthreads();
     if (!*last_flag) return;
     for (int t = wave; t < R * H; t += kWaves) {
         float4_t sum = {0.f, 0.f, 0.f, 0.f};
-        for (int s0 = 0; s0 < p.splits; s0 += 4) {
+        for (int s0 = 0; s0 < (int)splits; s0 += 4) {
             uint64_t v[4][2];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const uint64_t* ip = reinterpret_cast<const uint64_t*>(mine + ((int64_t)min(s0 + u, p.splits - 1) * (R * H) + t) * 256);
+                const uint64_t* ip = reinterpret_cast<const uint64_t*>(mine + ((int64_t)min(s0 + u, (int)splits - 1) * (R * H) + t) * 256);
                 v[u][0] = __hip_atomic_load(ip, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 v[u][1] = __hip_atomic_load(ip + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                if (s0 + u < p.splits) {
+                if (s0 + u < (int)splits) {
                     sum[0] += lo_float(v[u][0]);
                     sum[1] += hi_float(v[u][0]);
                     sum[2] += lo_float(v[u][1]);
@@ -378,7 +399,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 }
 
 template<int R, int H, int NQ>
-hipError_t launch_one(const BatchParams& p, hipStream_t st)
+hipError_t launch_one(const BatchArgs& p, hipStream_t st)
 {
     auto                         kfn = batch_kernel<R, H, NQ>;
     constexpr int                lds = H * 32 * 1024;
@@ -387,7 +408,8 @@ hipError_t launch_one(const BatchParams& p, hipStream_t st)
         const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kfn), lds, raised);
         if (e != hipSuccess) return e;
     }
-    return launch_kernel(kfn, dim3(p.strips * p.tiles_t * p.splits), dim3(64 * kWaves), (size_t)lds, st, p);
+    return launch_kernel(kfn, dim3((p.strips * p.tiles_t) << (p.how & 0xff)), dim3(64 * kWaves), (size_t)lds, st, p.A, p.X, p.Q, p.N, p.T, p.K, p.strips,
+                         p.tiles_t, p.by_strips, p.by_tiles_t, p.how, p.C, p.Rsd, p.ws, p.cnt, p.epoch);
 }
 
 // the widths that exist: up to four column tiles, and six or eight while the accumulators leave room (a workgroup costs about as
@@ -399,7 +421,7 @@ constexpr bool width_exists(int r, int h)
 }
 
 template<int H, int NQ>
-hipError_t launch_r(int r, const BatchParams& p, hipStream_t st)
+hipError_t launch_r(int r, const BatchArgs& p, hipStream_t st)
 {
     switch (r) {
         case 1:
@@ -420,7 +442,7 @@ hipError_t launch_r(int r, const BatchParams& p, hipStream_t st)
 }
 
 template<int NQ>
-hipError_t launch_h(int r, int h, const BatchParams& p, hipStream_t st)
+hipError_t launch_h(int r, int h, const BatchArgs& p, hipStream_t st)
 {
     switch (h) {
         case 1: return launch_r<1, NQ>(r, p, st);
@@ -442,7 +464,7 @@ bool batch_feasible(const BatchConfig& cf, int N, int T, int K, size_t ws_bytes,
     if ((int64_t)T * K * 2 >= (1ll << 32)) return false;
     const int64_t tiles = (int64_t)((N / kTileN + cf.r - 1) / cf.r) * ((T + 16 * cf.h - 1) / (16 * cf.h));
     if (cf.splits > 1 && (K / kGroup < cf.splits || tiles > cnt_len || (int64_t)batch_scratch_bytes(cf, N, T) > (int64_t)ws_bytes)) return false;
-    return cf.splits >= 1 && tiles * cf.splits < (1ll << 31);
+    return (cf.splits == 1 || cf.splits == 2 || cf.splits == 4) && tiles * cf.splits < (1ll << 31);
 }
 
 size_t batch_scratch_bytes(const BatchConfig& cf, int N, int T)
@@ -459,8 +481,11 @@ int batch_grid(const BatchConfig& cf, int N, int T)
 hipError_t batch_launch(const BatchConfig& cf, int nq, const GemmArgs& a, const Scratch& sc, hipStream_t st)
 {
     if (cf.splits > 1 && (sc.ws == nullptr || sc.cnt == nullptr)) return hipErrorInvalidValue;
-    BatchParams p{a.C, reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.R, a.N, a.T, a.K, (a.N / kTileN + cf.r - 1) / cf.r,
-                  (a.T + 16 * cf.h - 1) / (16 * cf.h), cf.splits, a.epilogue, sc.ws, sc.cnt, sc.epoch};
+    const uint32_t strips = (uint32_t)((a.N / kTileN + cf.r - 1) / cf.r), tiles_t = (uint32_t)((a.T + 16 * cf.h - 1) / (16 * cf.h));
+    const uint32_t log_splits = cf.splits == 1 ? 0 : cf.splits == 2 ? 1 : 2;
+    const uint64_t rows = (uint64_t)strips << log_splits;
+    BatchArgs      p{reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.N, a.T, a.K, strips, tiles_t, reciprocal(rows, strips),
+                reciprocal(rows * tiles_t, tiles_t), log_splits | (uint32_t)a.epilogue << 8, a.C, a.R, sc.ws, sc.cnt, sc.epoch};
     switch (nq) {
         case 1: return launch_h<1>(cf.r, cf.h, p, st);
         case 2: return launch_h<2>(cf.r, cf.h, p, st);
