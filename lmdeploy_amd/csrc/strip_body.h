@@ -542,59 +542,69 @@ __device__ __forceinline__ void strip_body(const StripParams& p, int col0, u32x4
         });
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the masked refills of the last trip
+    static_for<0, D>([&](auto d) { pin(st[d]); });  // (whose registers are nobody else's until then)
 
-    // ---- add the eight slices in LDS, in slice order ----
+    // ---- add the slices in LDS, in slice order: a unit is four tokens of a tile, lane (i, c) of a wave takes column c of token i ----
+    // (One wave per tile, four tokens to a lane, was the first way: the last wave of a workgroup then ran sixteen 128-bit reads and
+    // four masked stores by itself, and for a residual a trip to memory in front of them, 1200 of a narrow kernel's 4700 cycles.
+    // us, 11008 x 4096 with a residual at 4 / 8 tokens 7.31 -> 6.75 / 8.13 -> 7.60, 4096 x 4096 at one 4.06 -> 3.88; group size 64
+    // at 4 tokens, four Llama-2-7B matrices 32.6 -> 31.2, group size 32 35.8 -> 34.0.)
+    constexpr int kQuads = TP < 16 ? TP / 4 : 4, kUnits = R * H * kQuads, kMine = (kUnits + NW - 1) / NW;
+    const int     epi = EPI == kEpiRuntime ? p.epilogue : EPI;
+    int           row[kMine], col[kMine];
+    uint16_t      res[kMine];  // (requested before the waves wait for each other)
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) {
+        const int u = wave + m * NW;
+        row[m]      = u / kQuads % H * 16 + u % kQuads * 4 + b;
+        col[m]      = (col0 + u / (kQuads * H)) * kTileN + c;
+        res[m]      = 0;
+        if (epi == kEpiAdd && u < kUnits && row[m] < Tl) {
+            const uint16_t* at = p.Rsd + (int64_t)(t0 + row[m]) * N + col[m];
+            if constexpr (SEQ) res[m] = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else res[m] = *at;
+        }
+    }
     // red[slice][r][h][lane] as float4, over the activation patches: every wave must be done with its own
     __syncthreads();
-    float4_t* red4 = reinterpret_cast<float4_t*>(smem);
+    if (4 * b < TP) {
+        float4_t* red4 = reinterpret_cast<float4_t*>(smem);
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+        for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int h = 0; h < H; ++h) red4[((wave * R + r) * H + h) * 64 + lane] = acc[h][r];
+            for (int h = 0; h < H; ++h) red4[((wave * R + r) * H + h) * 64 + lane] = acc[h][r];
+    }
     __syncthreads();
-    for (int rh = wave; rh < R * H; rh += NW) {  // (tile r, row block h) is finished by wave r * H + h (mod NW)
-        const int r = rh / H, h = rh % H;
-        float4_t  v = {0.f, 0.f, 0.f, 0.f};
+    const float* red = reinterpret_cast<const float*>(smem);
 #pragma unroll
-        for (int s = 0; s < NW; ++s) v += red4[((s * R + r) * H + h) * 64 + lane];
+    for (int m = 0; m < kMine; ++m) {
+        const int u = wave + m * NW;
+        if (u >= kUnits) break;
+        // (unit u of a slice: quad u % kQuads of the 64 lanes' float4 of tile and row block u / kQuads)
+        const float* from = red + (u / kQuads * 64 + u % kQuads * 16 + c) * 4 + b;
+        float        v    = 0.f;
+#pragma unroll
+        for (int s = 0; s < NW; ++s) v += from[s * (R * H * 256)];
 
-        // ---- epilogue: lane (c, b) holds column n = 16 * (col0 + r) + c, tokens t0 + 16h + 4b + i ----
-        const int n   = (col0 + r) * kTileN + c;
-        const int epi = EPI == kEpiRuntime ? p.epilogue : EPI;
+        // ---- epilogue ----
+        const half_t hv    = (half_t)v;
+        const int    token = t0 + row[m], n = col[m];
+        const bool   in    = row[m] < Tl;
         auto put = [&](int64_t at, half_t o) {
             const uint16_t bits = __builtin_bit_cast(uint16_t, o);
             if constexpr (SEQ) __hip_atomic_store(p.C + at, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             else p.C[at] = bits;
         };
-        // (the four residual loads of a lane are issued together: at agent scope each is a trip to memory)
-        uint16_t rb[4] = {0, 0, 0, 0};
-        if (epi == kEpiAdd) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = 16 * h + 4 * b + i;
-                if (row < Tl) {
-                    const int64_t at = (int64_t)(t0 + row) * N + n;
-                    if constexpr (SEQ) rb[i] = __hip_atomic_load(p.Rsd + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    else rb[i] = p.Rsd[at];
-                }
-            }
+        if (epi == kEpiSilu) {
+            // gate = even column, up = odd column: fetch the neighbour lane's value
+            const float mine  = (float)hv;
+            const float other = __shfl_xor(mine, 1);
+            if (in && (c & 1) == 0) put((int64_t)token * (N / 2) + (n >> 1), (half_t)(mine / (1.f + __expf(-mine)) * other));
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const half_t hv    = (half_t)v[i];
-            const int    row   = 16 * h + 4 * b + i;
-            const int    token = t0 + row;
-            if (epi == kEpiSilu) {
-                // gate = even column, up = odd column: fetch the neighbour lane's value
-                const float mine  = (float)hv;
-                const float other = __shfl_xor(mine, 1);
-                if (row < Tl && (c & 1) == 0) put((int64_t)token * (N / 2) + (n >> 1), (half_t)(mine / (1.f + __expf(-mine)) * other));
-            }
-            else if (row < Tl) {
-                const int64_t at = (int64_t)token * N + n;
-                if (epi == kEpiGemm) put(at, hv);
-                else put(at, (half_t)((float)__builtin_bit_cast(half_t, rb[i]) + (float)hv));
-            }
+        else if (in) {
+            const int64_t at = (int64_t)token * N + n;
+            if (epi == kEpiGemm) put(at, hv);
+            else put(at, (half_t)((float)__builtin_bit_cast(half_t, res[m]) + (float)hv));
         }
     }
 }
