@@ -301,7 +301,87 @@ batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int 
         step(S1{}, no{}, no{});
     }
 
-    const int epi  = (int)(how >> 8);
+    const int    epi  = (int)(how >> 8);
+    const int    tile = (int)(strip * tiles_t + tile_t);
+    float4_t*    red4 = reinterpret_cast<float4_t*>(smem);
+    const float* red  = reinterpret_cast<const float*>(smem);
+    // split K, as in the tile kernels: stores through to memory, an arrival counter, the last one adds
+    auto last_to_arrive = [&]() {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        int* const last_flag = reinterpret_cast<int*>(smem);
+        if (tid == 0) {
+            const bool last = arrive_last(counters + tile, (int)splits, epoch);
+            *last_flag = last;
+        }
+        __syncthreads();
+        return *last_flag != 0;
+    };
+    // One or two tiles of sums are shared out by units of four tokens, more of them by tiles: a wave that adds up a whole tile
+    // stores eight bytes to a lane, where units store two, but with fewer tiles than waves it is what everything waits for (us,
+    // tiles and units, 16 tokens: 8192 x 1024 split in four 6.20 and 5.77; 48 tokens: 4096 x 12288 11.65 and 11.85).
+    if constexpr (R * H <= 2) {
+        // lane (i, c) of a unit takes column c of token i
+        auto      emit = [&](int u, float v, uint16_t res) {
+            const int    token = t0 + u / 4 % H * 16 + u % 4 * 4 + b, r = u / (4 * H), n = (col0 + r) * kTileN + c;
+            const half_t hv = (half_t)v;
+            const bool   in = token < T && col0 + r >= first;
+            if (epi == kEpiSilu) {  // gate = even column, up = odd column
+                const float mine = (float)hv, other = __shfl_xor(mine, 1);
+                float        y = mine / (1.f + __expf(-mine)) * other;
+                asm volatile("" : "+v"(y));  // (rounded to fp32 and then to fp16, as everywhere: one instruction could do both)
+                const half_t o = (half_t)y;
+                if (in && (c & 1) == 0) C[(int64_t)token * (N / 2) + (n >> 1)] = __builtin_bit_cast(uint16_t, o);
+            }
+            else if (in) {
+                const half_t o = epi == kEpiAdd ? (half_t)((float)__builtin_bit_cast(half_t, res) + (float)hv) : hv;
+                C[(int64_t)token * N + n] = __builtin_bit_cast(uint16_t, o);
+            }
+        };
+        auto residual = [&](int u) -> uint16_t {
+            const int token = t0 + u / 4 % H * 16 + u % 4 * 4 + b, r = u / (4 * H);
+            return token < T ? Rsd[(int64_t)token * N + (col0 + r) * kTileN + c] : (uint16_t)0;
+        };
+        constexpr int kUnits = R * H * 4, kMine = (kUnits + kWaves - 1) / kWaves;
+        float* const  mine = ws + ((int64_t)tile * (int)splits) * (kUnits * 64) + lane;
+        uint16_t      res[kMine];  // (requested before the waves wait for each other)
+#pragma unroll
+        for (int m = 0; m < kMine; ++m) res[m] = epi == kEpiAdd && splits == 1 && wave + m * kWaves < kUnits ? residual(wave + m * kWaves) : (uint16_t)0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int h = 0; h < H; ++h) red4[((wave * R + r) * H + h) * 64 + lane] = acc[r][h];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < kMine; ++m) {
+            const int u = wave + m * kWaves;
+            if (u >= kUnits) break;
+            const float* from = red + (u / 4 * 64 + u % 4 * 16 + c) * 4 + b;
+            float        v    = 0.f;
+#pragma unroll
+            for (int s = 0; s < kWaves; ++s) v += from[s * (R * H * 256)];
+            if (splits == 1) emit(u, v, res[m]);
+            else __hip_atomic_store(mine + ((int64_t)(int)split * kUnits + u) * 64, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (splits == 1 || !last_to_arrive()) return;
+#pragma unroll
+        for (int m = 0; m < kMine; ++m) {
+            const int u = wave + m * kWaves;
+            if (u >= kUnits) break;
+            float part[4];  // of up to four splits
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+                part[z] = __hip_atomic_load(mine + ((int64_t)min(z, (int)splits - 1) * kUnits + u) * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint16_t rs  = epi == kEpiAdd ? residual(u) : (uint16_t)0;
+            float          sum = 0.f;
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+                if (z < (int)splits) sum += part[z];
+            emit(u, sum, rs);
+        }
+        return;
+    }
     auto      emit = [&](int r, int h, const float4_t v) {  // lane (c, b): token t0 + 16h + c, features n .. n + 3
         const int token = t0 + 16 * h + c;
         if (token >= T || col0 + r < first) return;
@@ -334,9 +414,6 @@ batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int 
 #pragma unroll
     for (int i = 0; i < 4; ++i) get_at[i] = (16 * (c >> 2) + ((4 * b + i) ^ (c >> 2))) * 4 + (c & 3);
     constexpr int RC   = R < 4 ? R : 4;
-    float4_t*     red4 = reinterpret_cast<float4_t*>(smem);
-    const float*  red  = reinterpret_cast<const float*>(smem);
-    const int     tile = (int)(strip * tiles_t + tile_t);
     float* const  mine = ws + ((int64_t)tile * (int)splits) * (R * H) * 256 + lane * 4;
 #pragma unroll
     for (int r0 = 0; r0 < R; r0 += RC) {
@@ -363,18 +440,7 @@ batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int 
             }
         }
     }
-    if ((int)splits == 1) return;
-
-    // ---- split K: as in the tile kernels, stores through to memory, an arrival counter, the last one adds ----
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    int* const last_flag = reinterpret_cast<int*>(smem);
-    if (tid == 0) {
-        const bool last = arrive_last(counters + tile, (int)splits, epoch);
-        *last_flag = last;
-    }
-    __syncthreads();
-    if (!*last_flag) return;
+    if (splits == 1 || !last_to_arrive()) return;
     for (int t = wave; t < R * H; t += kWaves) {
         float4_t sum = {0.f, 0.f, 0.f, 0.f};
         for (int s0 = 0; s0 < (int)splits; s0 += 4) {
