@@ -16,11 +16,12 @@ namespace w4a16 {
 
 namespace {
 
-constexpr size_t kCounterBytes = kStaticCounters * sizeof(int);
+constexpr size_t kCounterBytes = 2 * kStaticCounters * sizeof(int);
 constexpr size_t kStaticBytes  = kCounterBytes + kStaticWorkspaceBytes;
 constexpr int    kMaxDevices   = 64;
 
-// [arrival counters: kStaticCounters ints][fp32 partial tiles: kStaticWorkspaceBytes]
+// [arrival counters: kStaticCounters ints][the second ones, for counts that did not start from zero (arrive_last): as many]
+// [fp32 partial tiles: kStaticWorkspaceBytes]
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];
 
 std::mutex     g_mutex;
@@ -71,9 +72,7 @@ hipError_t static_scratch(Scratch* out)
 // Before a launch that counts arrivals in `sc`, of static_scratch, with `n` counters.  A launch made at once has a tag that no
 // earlier one used, and starts from whatever is there.  The replays of a recorded launch all carry one tag, and a count that
 // overlapping calls left under it would be taken for the replay's own, each time: there the counters are cleared first, by a
-// kernel (not hipMemsetAsync, whose nodes a graph may replay wrongly), and counted without a tag.  8192 x 1024 at 16 tokens, K
-// split in four: in a graph 9.1 us a launch with tags, 7.9 with the clearing kernel and without; made at once 8.0 with tags, 8.4
-// with the clearing kernel, which is a second call for the host to make.
+// kernel (not hipMemsetAsync, whose nodes a graph may replay wrongly), and counted without a tag.
 hipError_t prepare_static_counters(Scratch* sc, int n, hipStream_t st)
 {
     // (the null stream cannot be captured, and must not be asked while another one is)

@@ -76,3 +76,32 @@ def test_counts_left_behind_concern_no_later_launch_or_replay(K, N, T, kind):
             tm.gemm_static(E, A, X, Q, N, T, K, 128, 0, algo)
             torch.cuda.synchronize()
             assert torch.equal(E.view(torch.int16), H.view(torch.int16)), ("call", algo, word >> TAG_SHIFT, word & 4095)
+
+
+@pytest.mark.parametrize("splits_of", [(8192, 1024, 16), (4224, 1024, 100)])
+def test_second_counters_left_behind(splits_of):
+    """A count that did not start from zero is taken on a second set of counters: whatever those hold, and the call after it."""
+    import lmdeploy_amd.turbomind as tm
+    from lmdeploy_amd._lib import lib
+    K, N, T = splits_of
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    words = lambda *size: torch.randint(-2 ** 31, 2 ** 31, size, dtype=torch.int32, device="cuda", generator=gen)
+    s = (torch.randn((K // 128, N), device="cuda", generator=gen).abs() * 0.01 + 1e-3).half()
+    qw = words(K, N // 8)
+    A, Q = torch.empty_like(qw), torch.empty_like(s, dtype=torch.int32)
+    tm.convert_s4_k_m8(A, Q, s, qw, s, words(K // 128, N // 8), N, K, 128)
+    X, H, E = torch.randn((T, K), device="cuda", generator=gen).half(), *torch.empty((2, T, N), dtype=torch.float16, device="cuda")
+    gemm = tm.GemmS4F16()
+    gemm.Run(H, A, X, Q, N, T, K, 128)
+    fn = lib.hipMemcpy
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+    for first, second in ((0, 3), (3, 0), (3, 3), (1 << 20, -1), (-1, 2 << TAG_SHIFT | 1)):
+        at = scratch(lib)
+        both = (ctypes.c_int * (2 * at.cnt_len))(*([first] * at.cnt_len + [second] * at.cnt_len))
+        torch.cuda.synchronize()
+        assert fn(at.cnt, both, 8 * at.cnt_len, 1) == 0
+        for call in range(3):
+            E.fill_(float("nan"))
+            tm.gemm_static(E, A, X, Q, N, T, K, 128)
+            torch.cuda.synchronize()
+            assert torch.equal(E.view(torch.int16), H.view(torch.int16)), (first, second, call)
