@@ -48,19 +48,6 @@ struct BatchArgs {
     int             epoch;
 };
 
-// n / d for n below some bound: d == 1 has the reciprocal 0, the others floor(2^32 / d) + 1 (exact while n d < 2^32, Granlund
-// and Montgomery), or 1 where the bound does not allow that and n is divided by d.
-uint32_t reciprocal(uint64_t bound, uint32_t d)
-{
-    return d == 1 ? 0 : bound * d < (1ull << 32) ? (uint32_t)((1ull << 32) / d) + 1 : 1;
-}
-__device__ __forceinline__ uint32_t divide_by(uint32_t n, uint32_t d, uint32_t reciprocal)
-{
-    if (reciprocal == 0) return n;
-    if (reciprocal == 1) return n / d;
-    return __umulhi(n, reciprocal);
-}
-
 // Loads of the software pipeline, waited for by count.  Their outputs are not tied to the value they replace: nothing
 // reads a stage between its refill and its wait, and the register allocator then has no reason to move a value whose
 // load is in flight (the build checks that it does not).
@@ -548,7 +535,7 @@ hipError_t batch_launch(const BatchConfig& cf, int nq, const GemmArgs& a, const 
 {
     if (cf.splits > 1 && (sc.ws == nullptr || sc.cnt == nullptr)) return hipErrorInvalidValue;
     const uint32_t strips = (uint32_t)((a.N / kTileN + cf.r - 1) / cf.r), tiles_t = (uint32_t)((a.T + 16 * cf.h - 1) / (16 * cf.h));
-    const uint32_t log_splits = cf.splits == 1 ? 0 : cf.splits == 2 ? 1 : 2;
+    const uint32_t log_splits = (uint32_t)log2_of(cf.splits);
     const uint64_t rows = (uint64_t)strips << log_splits;
     BatchArgs      p{reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.N, a.T, a.K, strips, tiles_t, reciprocal(rows, strips),
                 reciprocal(rows * tiles_t, tiles_t), log_splits | (uint32_t)a.epilogue << 8, a.C, a.R, sc.ws, sc.cnt, sc.epoch};

@@ -58,9 +58,8 @@ __device__ __forceinline__ void wait_lgkm0(half8_t& a, half8_t& b, half8_t& c, h
 // double the cover at the price of a second set of fragment registers.
 template<int TTILES, int NTW, int WAVES, int D, int KS, int EPI>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
-prefill_kernel(uint16_t* __restrict__ C, const u32x4_t* __restrict__ A, const uint16_t* __restrict__ X,
-               const uint32_t* __restrict__ Q, const uint16_t* R_, int N, int T, int K, int tiles_t, int tiles_n,
-               float* ws, int* cnt, int epoch)
+prefill_kernel(const u32x4_t* __restrict__ A, const uint16_t* __restrict__ X, const uint32_t* __restrict__ Q, int N, int T, int K, int tiles_t,
+               int tiles_n, uint32_t by_divisor, uint32_t log_splits, uint16_t* __restrict__ C, const uint16_t* R_, float* ws, int* cnt, int epoch)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [D][TT][kRowBytes]
     constexpr int TT = 16 * TTILES;
@@ -76,34 +75,14 @@ prefill_kernel(uint16_t* __restrict__ C, const u32x4_t* __restrict__ A, const ui
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c    = lane & 15;
     const int b    = lane >> 4;
-    const int G    = K / kGroup;
-    const int NT   = N / kTileN;
-
-    // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a contiguous run of tiles so
-    // its private L2 sees the reuse.  Inside a run, tiles go four token tiles at a time across
-    // the feature tiles: the ~64 workgroups an XCD runs concurrently then cover 4 token tiles x
-    // 16 feature tiles, which minimises what they fetch together (a token tile of activations
-    // is four times larger than a feature tile of int4 weights).
+    const int G    = (int)((uint32_t)K / kGroup);
+    const int NT   = (int)((uint32_t)N / kTileN);
     const int total = tiles_t * tiles_n;
     int       id    = blockIdx.x;
     if (total % 8 == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-    int tile_t, tile_n;
-    if (tiles_t % 4 == 0) {
-        const int r = id >> 2;
-        tile_n      = r % tiles_n;
-        tile_t      = (r / tiles_n) * 4 + (id & 3);
-    }
-    else {
-        tile_t = id % tiles_t;
-        tile_n = id / tiles_t;
-    }
-    // split K: blockIdx.y takes the quantisation groups [gbeg, gend), dealt in pairs so that only
-    // the last split can have an odd number of them
-    const int splits = gridDim.y;
-    const int pairs  = (G + 1) / 2;
-    const int gbeg   = min(G, 2 * (int)((int64_t)pairs * blockIdx.y / splits));
-    const int gend   = min(G, 2 * (int)((int64_t)pairs * (blockIdx.y + 1) / splits));
-    const int T0     = tile_t * TT;
+    const TilePlace at     = tile_place(id, tiles_t, tiles_n, by_divisor, G, (int)blockIdx.y, (int)log_splits);
+    const int       splits = 1 << log_splits, tile_n = at.tile_n, gbeg = at.gbeg, gend = at.gend;
+    const int       T0     = at.tile_t * TT;
     const int nt0    = (tile_n * TN) / kTileN + wave * NTW;  // first weight tile of this wave
 
     // per-thread byte offsets; the group-dependent part of every address is scalar
@@ -467,14 +446,15 @@ hipError_t launch_v(int splits, const GemmArgs& a, const Scratch& sc, hipStream_
     const size_t  lds     = (size_t)D * TT * kRowBytes;
     const dim3    grid(tiles_t * tiles_n, splits), block(64 * WAVES);
     const u32x4_t* A4 = reinterpret_cast<const u32x4_t*>(a.A);
+    const uint32_t by = reciprocal((uint64_t)tiles_t * tiles_n, tile_divisor(tiles_t, tiles_n));
 #define W4A16_LAUNCH(EPI)                                                                                              \
     do {                                                                                                               \
         auto                         kfn = prefill_kernel<TTILES, NTW, WAVES, D, KS, EPI>;                             \
         static std::atomic<uint64_t> raised{0}; /* per instantiation, one bit per device */                            \
         const hipError_t             e = raise_lds_limit(reinterpret_cast<const void*>(kfn), (int)lds, raised);        \
         if (e != hipSuccess) return e;                                                                                 \
-        return launch_kernel(kfn, grid, block, lds, st, a.C, A4, a.X, a.Q, a.R, a.N, a.T, a.K, tiles_t, tiles_n,       \
-                             sc.ws, sc.cnt, sc.epoch);                                                                      \
+        return launch_kernel(kfn, grid, block, lds, st, A4, a.X, a.Q, a.N, a.T, a.K, tiles_t, tiles_n, by,             \
+                             (uint32_t)log2_of(splits), a.C, a.R, sc.ws, sc.cnt, sc.epoch);                            \
     } while (0)
     switch (a.epilogue) {
         case kEpiGemm: W4A16_LAUNCH(kEpiGemm);
@@ -515,7 +495,7 @@ bool prefill_feasible(int v, int splits, int N, int T, int K, size_t ws_bytes, i
     const int64_t grid = (int64_t)(N / tn) * ((T + tt - 1) / tt);
     if (splits > 1) {
         // at least two groups per split; partial tiles and counters must fit the handle's scratch
-        if (K / kGroup < 2 * splits || splits > 65535) return false;
+        if (K / kGroup < 2 * splits || splits > 8 || (splits & (splits - 1)) != 0) return false;
         if (grid * splits * tn * tt * 4 > (int64_t)ws_bytes || grid > cnt_len) return false;
     }
     return grid * splits < (1ll << 31);

@@ -65,9 +65,9 @@ __device__ __forceinline__ float silu_quotient(float g)
 // 8..15 and 24..31; which rows of K a fragment covers does not matter as long as the activation fragment has the same.
 template<int TTILES, int NTW, int D, int NQ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-tile_kernel(uint16_t* __restrict__ C, const u32x4_t* __restrict__ A, const uint16_t* __restrict__ X,
-            const uint32_t* __restrict__ Q, const uint16_t* R_, int N, int T, int K, int tiles_t, int tiles_n, int epi,
-            float* ws, int* cnt, int epoch)
+tile_kernel(const u32x4_t* __restrict__ A, const uint16_t* __restrict__ X, const uint32_t* __restrict__ Q, int N, int T, int K, int tiles_t,
+            int tiles_n, uint32_t by_divisor, uint32_t how /* log2 of the K splits (8 bits), epilogue */, uint16_t* __restrict__ C,
+            const uint16_t* R_, float* ws, int* cnt, int epoch)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [D][4 TTILES][kBlock]
     constexpr int WAVES = 4;
@@ -84,32 +84,15 @@ tile_kernel(uint16_t* __restrict__ C, const u32x4_t* __restrict__ A, const uint1
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c    = lane & 31;
     const int hi   = lane >> 5;
-    const int G    = K / kGroup;
-    const int NT   = N / kTileN;
-
-    // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a contiguous run of tiles so
-    // its private L2 sees the reuse.  Inside a run, tiles go four token tiles at a time across
-    // the feature tiles.
+    const int G    = (int)((uint32_t)K / kGroup);
+    const int NT   = (int)((uint32_t)N / kTileN);
     const int total = tiles_t * tiles_n;
     int       id    = blockIdx.x;
     if (total % 8 == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-    int tile_t, tile_n;
-    if (tiles_t % 4 == 0) {
-        const int r = id >> 2;
-        tile_n      = r % tiles_n;
-        tile_t      = (r / tiles_n) * 4 + (id & 3);
-    }
-    else {
-        tile_t = id % tiles_t;
-        tile_n = id / tiles_t;
-    }
-    // split K: blockIdx.y takes the quantisation groups [gbeg, gend), dealt in pairs so that only
-    // the last split can have an odd number of them
-    const int splits = gridDim.y;
-    const int pairs  = (G + 1) / 2;
-    const int gbeg   = min(G, 2 * (int)((int64_t)pairs * blockIdx.y / splits));
-    const int gend   = min(G, 2 * (int)((int64_t)pairs * (blockIdx.y + 1) / splits));
-    const int T0     = tile_t * TT;
+    const int       log_splits = (int)(how & 0xff), splits = 1 << log_splits, epi = (int)(how >> 8);
+    const TilePlace at = tile_place(id, tiles_t, tiles_n, by_divisor, G, (int)blockIdx.y, log_splits);
+    const int       tile_n = at.tile_n, gbeg = at.gbeg, gend = at.gend;
+    const int       T0 = at.tile_t * TT;
     // this wave's weight tiles; at the right edge they overlap the neighbour's, which then owns those below `first`
     const int first = (tile_n * WAVES + wave) * NTW;
     const int nt0   = min(first, NT - NTW);
@@ -510,8 +493,10 @@ hipError_t launch_tile_one(int splits, const GemmArgs& a, const Scratch& sc, hip
     static std::atomic<uint64_t> raised{0};  // per instantiation, one bit per device
     const hipError_t             e = raise_lds_limit(reinterpret_cast<const void*>(kfn), (int)lds, raised);
     if (e != hipSuccess) return e;
-    return launch_kernel(kfn, dim3(tiles_t * tiles_n, splits), dim3(256), lds, st, a.C, reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q,
-                         a.R, a.N, a.T, a.K, tiles_t, tiles_n, a.epilogue, sc.ws, sc.cnt, sc.epoch);
+    const uint32_t how = (uint32_t)log2_of(splits) | (uint32_t)a.epilogue << 8;
+    return launch_kernel(kfn, dim3(tiles_t * tiles_n, splits), dim3(256), lds, st, reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.N, a.T, a.K,
+                         tiles_t, tiles_n, reciprocal((uint64_t)tiles_t * tiles_n, tile_divisor(tiles_t, tiles_n)), how, a.C, a.R, sc.ws, sc.cnt,
+                         sc.epoch);
 }
 
 // The tiles that exist (api.cpp has their prices), stages by what LDS holds.

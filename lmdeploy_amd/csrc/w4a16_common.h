@@ -157,6 +157,48 @@ __device__ __forceinline__ void spread_q(uint32_t x, uint32_t* q)
     }
 }
 
+// n / d for n below some bound: d == 1 has the reciprocal 0, the others floor(2^32 / d) + 1 (exact while n d < 2^32, Granlund
+// and Montgomery), or 1 where the bound does not allow that and n is divided by d.
+inline uint32_t reciprocal(uint64_t bound, uint32_t d)
+{
+    return d == 1 ? 0 : bound * d < (1ull << 32) ? (uint32_t)((1ull << 32) / d) + 1 : 1;
+}
+__device__ __forceinline__ uint32_t divide_by(uint32_t n, uint32_t d, uint32_t reciprocal)
+{
+    if (reciprocal == 0) return n;
+    if (reciprocal == 1) return n / d;
+    return __umulhi(n, reciprocal);
+}
+
+// The place of a workgroup of the MFMA tile kernels: which tile, and which quantisation groups of K.  Workgroups are dealt
+// round-robin to the 8 XCDs; each XCD gets a contiguous run of tiles, so that its private L2 sees the reuse.  Inside a run, tiles
+// go four token tiles at a time across the feature tiles: the ~64 workgroups an XCD runs concurrently then cover 4 token tiles x 16
+// feature tiles, which minimises what they fetch together (a token tile of activations is four times larger than a feature tile
+// of int4 weights).  split K: the groups are dealt in pairs, so that only the last split can have an odd number of them.
+inline int log2_of(int splits) { return splits >= 8 ? 3 : splits >= 4 ? 2 : splits >= 2 ? 1 : 0; }
+struct TilePlace {
+    int tile_t, tile_n, gbeg, gend;
+};
+// what the tiles are divided by on the way, for `reciprocal`
+inline uint32_t tile_divisor(int tiles_t, int tiles_n) { return (uint32_t)(tiles_t % 4 == 0 ? tiles_n : tiles_t); }
+__device__ __forceinline__ TilePlace tile_place(int id, int tiles_t, int tiles_n, uint32_t by_divisor, int G, int split, int log_splits)
+{
+    TilePlace p;
+    if (tiles_t % 4 == 0) {
+        const int r = id >> 2, q = (int)divide_by((uint32_t)r, (uint32_t)tiles_n, by_divisor);
+        p.tile_n = r - q * tiles_n;
+        p.tile_t = q * 4 + (id & 3);
+    }
+    else {
+        p.tile_n = (int)divide_by((uint32_t)id, (uint32_t)tiles_t, by_divisor);
+        p.tile_t = id - p.tile_n * tiles_t;
+    }
+    const uint32_t pairs = ((uint32_t)G + 1) / 2;  // (K below 2^31: times eight splits in 32 bits)
+    p.gbeg = min(G, 2 * (int)(pairs * (uint32_t)split >> log_splits));
+    p.gend = min(G, 2 * (int)(pairs * (uint32_t)(split + 1) >> log_splits));
+    return p;
+}
+
 // Split K: a workgroup announces that its partial tile is complete; true for the last of `splits`, which leaves the counter
 // at zero for the next launch.  epoch 0: the counters belong to a handle, which nobody else touches, or were cleared right before
 // this launch.  Otherwise they are shared by every caller on the GPU, and launches that overlapped against the rules may have left
