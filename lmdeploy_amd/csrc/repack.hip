@@ -100,10 +100,11 @@ __global__ void __launch_bounds__(kThreads) deploy_q_kernel(uint32_t* __restrict
 // word (one column, 8 rows) lies a transposition of 8 x 8 nibbles, and because the tiled layout orders rows inside a
 // word as AWQ orders columns, it is a plain one: nibble p of output q = nibble q of input p, inputs and outputs taken
 // in AWQ order.  One thread reads the 32 words that one source word column holds for its quarter (b) of the tile's
-// rows - coalesced over the lanes, all in flight together -, transposes them in registers and writes eight 16-byte
-// vectors, 128 contiguous bytes; the (zero, scale) words ride in the same launch.  Bound by HBM: every byte is read and
-// written once.  The four matrices of a Llama-2-7B layer (212 MB moved): 61 us, 3.5 TB/s, where one gather of eight
-// words per destination word plus a launch for the (zero, scale) words took 214 us.
+// rows - coalesced over the lanes, all in flight together -, transposes them in registers and holds eight 16-byte
+// vectors, which lanes exchange through LDS so that a store covers 256 contiguous bytes of four tiles; the (zero, scale) words
+// ride in the same launch.  Bound by HBM: every byte is read and written once.  Stored as the threads held them, sixteen bytes
+// in each of 64 cache lines at a time, the weights kept the L2s busy with requests: Llama-2-70B's four matrices (899 MB moved)
+// 222.6 us, 4.0 TB/s, exchanged first 178, and with non-temporal stores 168.8, 5.3 TB/s (a device copy reaches 5.15).
 struct TilePair {
     const uint32_t* qw[2];  // the two word columns of the tile
     const uint32_t* qz[2];
@@ -167,13 +168,14 @@ __global__ void __launch_bounds__(kThreads)
 convert_tiles_kernel(uint32_t* __restrict__ dst, uint32_t* __restrict__ Q, const ColumnSource cs, int NT, int G,
                      int w_across, int w_blocks, int q_across)
 {
-    const int tid = threadIdx.x;
+    __shared__ u32x4_t exchange[4][512];  // one part for each wave, which waits for nobody else
+    const int          tid = threadIdx.x;
     if ((int)blockIdx.x < w_blocks) {
-        const int kt = blockIdx.x / w_across;
-        const int at = (blockIdx.x % w_across) * 64 + (tid & 63);  // word column: tile at / 2, word at % 2
-        const int b  = tid >> 6;
-        if (at >= 2 * NT) return;
-        const int       nt = at >> 1, h = at & 1;
+        const int kt   = blockIdx.x / w_across;
+        const int base = (blockIdx.x % w_across) * 64;  // first word column: tile base / 2
+        const int lane = tid & 63, b = tid >> 6;
+        const int at   = min(base + lane, 2 * NT - 1);  // word column: tile at / 2, word at % 2
+        const int nt = at >> 1, h = at & 1;
         const TilePair  t  = locate_tile(cs, nt);
         const uint32_t* p  = (h ? t.qw[1] : t.qw[0]) + (int64_t)(kt * kGroup + 8 * b) * (h ? t.ld[1] : t.ld[0]);
         const int       ld = h ? t.ld[1] : t.ld[0];
@@ -184,11 +186,23 @@ convert_tiles_kernel(uint32_t* __restrict__ dst, uint32_t* __restrict__ Q, const
             for (int e = 0; e < 8; ++e) in[j][e] = __builtin_nontemporal_load(p + (int64_t)(32 * j + row_of_nibble(e)) * ld);
 #pragma unroll
         for (int j = 0; j < 4; ++j) transpose_nibbles(in[j]);
-        u32x4_t* const out = reinterpret_cast<u32x4_t*>(dst) + ((int64_t)kt * NT + nt) * 64 + b * 16;
+        // A thread has eight 16-byte vectors of one tile, a store instruction should have 256 contiguous bytes (this wave's quarter)
+        // of four: they change places in the wave's part of LDS.  Vector v of tile t is at position v ^ g(t): the sixteen lanes
+        // that LDS serves together, two of eight tiles each or all of one, then touch every bank once, whichever way columns run.
+        const auto  g   = [](int tile) { return (tile & 7) | (tile & 1) << 3; };
+        u32x4_t* const mine = exchange[b];
+        const int   tl = lane >> 1;
+        if (base + lane < 2 * NT)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int col = row_of_nibble(q);
-            out[t.turn ? 2 * col + h : 8 * h + col] = u32x4_t{in[0][q], in[1][q], in[2][q], in[3][q]};
+            for (int q = 0; q < 8; ++q) {
+                const int col = row_of_nibble(q);
+                mine[tl * 16 + ((t.turn ? 2 * col + h : 8 * h + col) ^ g(tl))] = u32x4_t{in[0][q], in[1][q], in[2][q], in[3][q]};
+            }
+        u32x4_t* const out = reinterpret_cast<u32x4_t*>(dst) + ((int64_t)kt * NT + (base >> 1)) * 64 + b * 16 + (lane & 15);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int tile = 4 * i + (lane >> 4);
+            if ((base >> 1) + tile < NT) __builtin_nontemporal_store(mine[tile * 16 + ((lane & 15) ^ g(tile))], out + tile * 64);
         }
         return;
     }

@@ -163,3 +163,18 @@ def test_fused_tensor_entry_points_equal_the_reference_steps_bit_for_bit(G):
     assert np.array_equal(Q.cpu().numpy().view(np.uint32), Q_ref)
     with pytest.raises(tm.W4A16Error):
         tm.deploy_qkv(tuple(map(dev, q)), tuple(map(dev, k)), tuple(map(dev, v)), 96, G)     # 256 is not a multiple of 96
+
+
+@pytest.mark.parametrize("tiles", [1, 2, 31, 33, 65, 96])
+def test_conversion_of_any_number_of_tiles(tiles):
+    """32 tiles of 16 columns change places at a time: numbers of them on both sides of that, side by side, against the oracle."""
+    import lmdeploy_amd.turbomind as tm
+    K, N = 384, 16 * tiles
+    d = O.make_inputs(tiles, 1, K, N)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).cuda()
+    qw, qz, s = dev(d["qweight"]), dev(d["qzeros"]), dev(d["scales"])
+    A, Q = torch.zeros((K + 128, N // 8), dtype=torch.int32, device="cuda"), torch.zeros((K // G, N), dtype=torch.int32, device="cuda")
+    tm.convert_s4_k_m8(A[:K], Q, s, qw, s, qz, N, K, G)
+    A_ref, Q_ref = O.convert_s4_k_m8(d["qweight"], d["scales"], d["qzeros"], N, K, G)
+    assert np.array_equal(A[:K].cpu().numpy().view(np.uint32).reshape(-1), A_ref) and not A[K:].any()
+    assert np.array_equal(Q.cpu().numpy().view(np.uint32), Q_ref)
