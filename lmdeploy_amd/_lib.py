@@ -11,7 +11,7 @@ from ctypes import (POINTER, Structure, c_char_p, c_double, c_float, c_int, c_lo
 # torch ships its own libamdhip64 and libw4a16.so has to bind to that same HIP runtime.  Loaded the
 # other way round, the system runtime gets in first, two runtimes share the process, and the first
 # kernel launch reports "no ROCm-capable device is detected".
-import torch  # noqa: F401  (imported for its side effect on the dynamic loader)
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # W4A16_LIB overrides the in-tree library (e.g. to try a differently tuned build)
@@ -93,6 +93,21 @@ def _load() -> ctypes.CDLL:
 
 
 lib = _load()
+
+
+def _bind():
+    """The calls of a decode step and of a layer's conversion without ctypes (csrc/binding.cpp), through the functions of the library loaded above."""
+    from . import _binding  # ImportError if it has not been built
+    at = lambda fn: ctypes.cast(fn, c_void_p).value
+    # torch's own accessors of the current device and of its current stream's handle: torch.cuda.current_stream() wraps
+    # the same two in a Stream object, which takes 2.9 us against 0.2 us - more than the whole C call below it
+    _binding.bind(*map(at, (lib.w4a16_gemm, lib.w4a16_gemm_static, lib.w4a16_ffn, lib.w4a16_convert_s4_k_m8,
+                            lib.w4a16_deploy_qkv, lib.w4a16_deploy_w13)),
+                  torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, torch.nn.Parameter)
+    return _binding
+
+
+binding = _bind()
 
 
 def check(code: int) -> int:

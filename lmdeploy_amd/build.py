@@ -1,4 +1,4 @@
-"""Builds libw4a16.so (HIP kernels for gfx950 + the C ABI) in-tree with hipcc.
+"""Builds libw4a16.so (HIP kernels for gfx950 + the C ABI) in-tree with hipcc, and the Python extension over it.
 
 Usage: python -m lmdeploy_amd.build            (or build_library() from Python)
 """
@@ -9,12 +9,14 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libw4a16.so")
+BINDING_PATH = os.path.join(HERE, "_binding.so")
 
 SOURCES = ["api.cpp", "rounding_domain.cpp", "repack.hip", "static_scratch.hip", "probe.hip", "gemm_decode.hip", "gemm_strip.hip", "gemm_strip_groups.hip",
            "gemm_sequence.hip", "gemm_prefill.hip", "gemm_batch.hip", "gemm_tile_g128.hip", "gemm_tile_g64.hip", "gemm_tile_g32.hip"]
@@ -116,6 +118,24 @@ def build_library(verbose: bool = True) -> str:
     return LIB_PATH
 
 
+def build_binding(verbose: bool = True) -> str:
+    """Compiles csrc/binding.cpp, host code against Python's and torch's headers; it finds the library at run time."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    tmp = BINDING_PATH + ".tmp"
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(), "-I", sysconfig.get_paths()["include"],
+           "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           os.path.join(CSRC, "binding.cpp"), "-o", tmp, "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building the Python extension failed:\n%s\n%s" % (r.stdout, r.stderr))
+    os.replace(tmp, BINDING_PATH)
+    if verbose:
+        print("built", BINDING_PATH)
+    return BINDING_PATH
+
+
 def check_headers(verbose: bool = True) -> str:
     """Compiles and links tests/cpp/llama_linear_dropin.cpp against the C++ front-end headers and
     the library: the proof that a LlamaLinear-shaped caller builds against them."""
@@ -137,5 +157,6 @@ def check_headers(verbose: bool = True) -> str:
 
 if __name__ == "__main__":
     build_library()
+    build_binding()
     check_headers()
     sys.exit(0)

@@ -49,7 +49,7 @@ def convert_awq_layer(get: Callable[[str], torch.Tensor], i: int, group_size: in
     def plain(prefix: str):
         qw, qz, s = awq(prefix)
         A, Q = torch.empty_like(qw), torch.empty_like(s, dtype=torch.int32)   # Q: half2 per (group, feature)
-        tm.convert_s4_k_m8(A, Q, torch.empty(0, device=qw.device), qw, s, qz, qw.size(-1) * 8, qw.size(0), group_size)
+        tm.convert_s4_k_m8(A, Q, None, qw, s, qz, qw.size(-1) * 8, qw.size(0), group_size)
         return A, Q
 
     att, mlp = "model.layers.%d.self_attn." % i, "model.layers.%d.mlp." % i

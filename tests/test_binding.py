@@ -1,0 +1,83 @@
+"""The calls that go from Python to the C ABI without ctypes: plain arguments give what the general path gives, and every other
+form is left to that path, with nothing done."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import lmdeploy_amd.turbomind as tm
+from lmdeploy_amd._lib import GemmDesc, W4A16Error, binding, lib
+from oracle import w4a16_oracle as O
+
+
+class Wrapped(torch.Tensor):
+    pass
+
+
+def test_other_forms_are_left_to_the_general_path():
+    good = [None, None, None, None, None, 128, 1, 128, 128, 0, -1, 0]
+    assert binding.gemm_static(*good) == lib.w4a16_gemm_static(*good) == -4  # (null pointers are refused)
+    assert binding.gemm(0, *good) == lib.w4a16_gemm(0, *good) == -4
+    for at, bad in [(0, torch.zeros(2)), (1, torch.zeros(2).as_subclass(Wrapped)), (2, 5), (5, 1.0), (6, np.int64(1)), (7, 1 << 31),
+                    (8, -(1 << 31) - 1), (9, ctypes.c_int(0)), (10, None), (11, ctypes.c_void_p(0)), (11, 1 << 64)]:
+        assert binding.gemm_static(*good[:at], bad, *good[at + 1:]) is None, (at, bad)
+    assert binding.gemm_static(*good[:-1]) is None and binding.ptr(torch.zeros(2)) is None
+    assert binding.ffn(0, *[None] * 8, 128, 128, 1.5, 128, 0) is None and binding.gemm(None, *good) is None
+    with pytest.raises(ValueError, match="live on the GPU"):
+        tm.gemm_static(torch.zeros(2), None, None, None, 128, 1, 128, 128)
+    with pytest.raises(ctypes.ArgumentError):
+        tm.gemm_static(None, None, None, None, 128, 1.0, 128, 128, stream=0)
+    with pytest.raises(W4A16Error, match="null"):
+        tm.gemm_static(None, None, None, None, 128, 1, 128, 128, stream=0)
+
+
+@pytest.mark.parametrize("count", [0, 1, 5])
+def test_descriptors(count):
+    gemms = [(None, None, None, None, 8 * i, -i, i % 3, None, i % 2 == 0) for i in range(count)]
+    arr = (GemmDesc * count)()
+    assert binding.describe(arr, gemms) is True and binding.describe(arr, tuple(gemms)) is True
+    for i, d in enumerate(arr):
+        assert (d.C, d.A, d.X, d.Q, d.R, d.n_out, d.k, d.epilogue, d.depends) == (None,) * 5 + (8 * i, -i, i % 3, int(i % 2 == 0))
+    assert binding.describe((GemmDesc * (count + 1))(), gemms) is None  # (a wrong number of them)
+    if count:
+        for bad in (gemms[-1][:8], list(gemms[-1]), gemms[-1][:4] + (1.0,) + gemms[-1][5:], (torch.zeros(1),) + gemms[-1][1:],
+                    gemms[-1][:8] + ("yes",)):
+            assert binding.describe(arr, gemms[:-1] + [bad]) is None, bad
+
+
+@pytest.mark.gpu
+def test_both_paths_give_the_same():
+    T, K, N, g = 3, 256, 128, 128
+    d = O.make_inputs(77, T, K, N, g, residual=True)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).cuda()
+    qw, qz, s, X, R = (dev(d[n]) for n in ("qweight", "qzeros", "scales", "X", "R"))
+    A, Q = torch.zeros_like(qw), torch.zeros_like(s, dtype=torch.int32)
+    tm.convert_s4_k_m8(A, Q, torch.zeros_like(s), qw, s, qz, N, K, g)
+    op = tm.GemmS4F16()
+    out = [torch.empty(T, N, dtype=torch.float16, device="cuda") for _ in range(7)]
+    other = lambda t: t.as_subclass(Wrapped)
+    at = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    op.Run(out[0], A, X, Q, N, T, K, g, 2, -1, residual=R)
+    op.Run(out[1], torch.nn.Parameter(A, requires_grad=False), X, Q, N, T, K, g, 2, residual=R)
+    op.Run(other(out[2]), A, other(X), Q, N, T, K, g, 2, residual=R)
+    op.Run(out[3], A, X, Q, N, ctypes.c_int(T), K, g, 2, residual=R, stream=at)
+    tm.gemm_static(out[4], A, X, Q, N, T, K, g, 2, residual=R)
+    tm.gemm_static(out[5], A, X, Q, N, T, K, g, 2, residual=other(R))
+    op.sequence([[out[6], A, X, Q, N, K, 2, R, False]], T, g)
+    torch.cuda.synchronize()
+    want = O.gemm_s4_f16(d["X"], d["qweight"], d["qzeros"], d["scales"], g, 2, d["R"])
+    assert O.max_abs_rel(out[0].cpu().numpy(), want) <= 1e-2
+    for o in out[1:]:
+        assert torch.equal(o, out[0])
+    A2, Q2 = torch.zeros_like(A), torch.zeros_like(Q)
+    tm.convert_s4_k_m8(other(A2), Q2, None, qw, other(s), qz, N, K, g)
+    assert torch.equal(A2, A) and torch.equal(Q2, Q)
+    plain, mixed = (qw, qz, s), (other(qw), qz, other(s))
+    for made in (tm.deploy_qkv(plain, plain, mixed, 128, g), tm.deploy_w13(plain, list(plain), g)):
+        want = tm.deploy_qkv(plain, plain, plain, 128, g) if made[0].size(-1) == 3 * N // 8 else tm.deploy_w13(plain, plain, g)
+        assert torch.equal(made[0], want[0]) and torch.equal(made[1], want[1])
+    with pytest.raises(ValueError, match="contiguous"):
+        op.Run(out[0], A, X.t(), Q, N, T, K, g)
+    with pytest.raises(RuntimeError):  # inside a transform a tensor has no address
+        torch.vmap(lambda x: op.Run(out[0], A, x, Q, N, T, K, g))(X.expand(2, T, K).contiguous())
