@@ -239,6 +239,13 @@ int w4a16_deploy_w13(uint32_t* A_dst, void* Q_dst, const uint32_t* w1_qweight, c
                      const uint32_t* w1_qzeros, const uint32_t* w3_qzeros, const void* w1_scales, const void* w3_scales,
                      int inter_size, int k, int group_size, void* stream);
 
+/* All matrices of a decoder layer in one launch, with the results of w4a16_deploy_qkv, w4a16_convert_s4_k_m8 (o), w4a16_deploy_w13
+ * and w4a16_convert_s4_k_m8 (down).  qweight, qzeros, scales and the widths n are those of q, k, v, o, gate, up, down (n of k
+ * and v, and of gate and up, are the same); A_dst, Q_dst and the rows k those of q|k|v, o, gate|up, down. */
+int w4a16_deploy_layer(uint32_t* const A_dst[4], void* const Q_dst[4], const uint32_t* const qweight[7],
+                       const uint32_t* const qzeros[7], const void* const scales[7], const int n[7], const int k[4],
+                       int size_per_head, int group_size, void* stream);
+
 /* reformat_s4_k_m8 (format.h:13, format.cu:69-75): the weight half of the conversion alone,
  * AWQ words [k, m/8] -> the tiled layout the GEMM kernels read (here the gfx950 one).
  * format.h:11 `reformat_s4_k8_m` is an unused alternative layout and has no counterpart. */

@@ -60,6 +60,7 @@ SIGNATURES = {
     "w4a16_deploy_qkv": (c_int, [c_void_p, c_void_p, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p)] + [c_int] * 5
                          + [c_void_p]),
     "w4a16_deploy_w13": (c_int, [c_void_p] * 8 + [c_int] * 3 + [c_void_p]),
+    "w4a16_deploy_layer": (c_int, [POINTER(c_void_p)] * 5 + [POINTER(c_int)] * 2 + [c_int] * 2 + [c_void_p]),
     "w4a16_reformat_s4_k_m8": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "w4a16_fuse_w1_w3_s4_k_m8": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "w4a16_transpose_qk_s4_k_m8_hf": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
@@ -102,7 +103,7 @@ def _bind():
     # torch's own accessors of the current device and of its current stream's handle: torch.cuda.current_stream() wraps
     # the same two in a Stream object, which takes 2.9 us against 0.2 us - more than the whole C call below it
     _binding.bind(*map(at, (lib.w4a16_gemm, lib.w4a16_gemm_static, lib.w4a16_ffn, lib.w4a16_convert_s4_k_m8,
-                            lib.w4a16_deploy_qkv, lib.w4a16_deploy_w13)),
+                            lib.w4a16_deploy_layer)),
                   torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, torch.nn.Parameter)
     return _binding
 

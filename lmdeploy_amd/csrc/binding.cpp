@@ -1,8 +1,8 @@
-// The calls of lmdeploy_amd/turbomind.py that a decode step or a layer's conversion makes, from Python to the C ABI without ctypes in between: each
-// tensor's checks and address, the current stream, and the call itself.  The kernel of a 4096 x 4096 matrix takes 3.3 us for one
+// The calls of lmdeploy_amd/turbomind.py that a decode step or a layer's conversion makes, from Python to the C ABI without ctypes
+// in between: each tensor's checks and address, the current stream, and the call itself.  The kernel of a 4096 x 4096 matrix takes 3.3 us for one
 // token; through ctypes and Python's accessors the host needed 4.9 us for such a call, and 3.9 this way, of which the runtime's launch
-// takes 2.3.  A descriptor of a sequence takes 0.04 us instead of 0.8: the 128 of a decode step of 32 layers 5 us instead of 98.  The conversion of a layer takes the host 38 us instead of 45
-// (half of it torch's allocations), which is what a small layer's conversion takes.
+// takes 2.3.  A descriptor of a sequence takes 0.04 us instead of 0.8: the 128 of a decode step of 32 layers 5 us instead of 98.
+// A small layer's conversion, which the host sets the time of, takes 30 us instead of 54 (in one launch instead of four).
 //
 // Each function takes plain arguments only: None or a contiguous GPU tensor whose type is torch.Tensor or torch.nn.Parameter
 // itself, and whole numbers that fit their C types.  For anything else it returns None without having done anything, and the caller
@@ -24,8 +24,7 @@ decltype(&w4a16_gemm)            fn_gemm;
 decltype(&w4a16_gemm_static)     fn_gemm_static;
 decltype(&w4a16_ffn)             fn_ffn;
 decltype(&w4a16_convert_s4_k_m8) fn_convert;
-decltype(&w4a16_deploy_qkv)      fn_deploy_qkv;
-decltype(&w4a16_deploy_w13)      fn_deploy_w13;
+decltype(&w4a16_deploy_layer)    fn_deploy_layer;
 PyObject *                       get_device, *get_stream, *parameter_type;  // torch's accessors, and torch.nn.Parameter
 
 // The address of a plain contiguous tensor on the GPU, nullptr for None
@@ -150,31 +149,29 @@ bool triples(PyObject* const* t, int count, uint32_t** qweight, uint32_t** qzero
     return true;
 }
 
-// (A, Q, q, k, v, n_q, n_kv, K, size_per_head, group_size)
-PyObject* deploy_qkv(PyObject*, PyObject* const* a, Py_ssize_t n)
+// (4 pairs (A, Q), 7 triples (qweight, qzeros, scales), 7 widths, 4 numbers of rows, size_per_head, group_size), tuples all of them
+PyObject* deploy_layer(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
-    void *    p[2], *scales[3], *st;
-    uint32_t *qweight[3], *qzeros[3];
-    int       v[5], rc;
-    if (n != 10 || !addresses(a, 2, p) || !triples(a + 2, 3, qweight, qzeros, scales) || !numbers(a + 5, 5, v) || !stream_of(Py_None, &st))
+    void *    Q[4], *scales[7], *p[3], *st;
+    uint32_t *dst[4], *qweight[7], *qzeros[7];
+    int       width[7], rows[4], v[2], rc;
+    auto      tuple = [](PyObject* o, Py_ssize_t size) { return PyTuple_CheckExact(o) && PyTuple_GET_SIZE(o) == size; };
+    bool      ok    = n == 6 && tuple(a[0], 4) && tuple(a[1], 7) && tuple(a[2], 7) && tuple(a[3], 4);
+    for (int i = 0; ok && i < 4; ++i) {
+        PyObject* const t = PyTuple_GET_ITEM(a[0], i);
+        ok                = tuple(t, 2) && addresses(PySequence_Fast_ITEMS(t), 2, p);
+        if (ok) dst[i] = static_cast<uint32_t*>(p[0]), Q[i] = p[1];
+    }
+    for (int i = 0; ok && i < 7; ++i) {
+        PyObject* const t = PyTuple_GET_ITEM(a[1], i);
+        ok                = tuple(t, 3) && addresses(PySequence_Fast_ITEMS(t), 3, p);
+        if (ok) qweight[i] = static_cast<uint32_t*>(p[0]), qzeros[i] = static_cast<uint32_t*>(p[1]), scales[i] = p[2];
+    }
+    if (!ok || !numbers(PySequence_Fast_ITEMS(a[2]), 7, width) || !numbers(PySequence_Fast_ITEMS(a[3]), 4, rows) || !numbers(a + 4, 2, v) ||
+        !stream_of(Py_None, &st))
         Py_RETURN_NONE;
     Py_BEGIN_ALLOW_THREADS;
-    rc = fn_deploy_qkv(static_cast<uint32_t*>(p[0]), p[1], qweight, qzeros, scales, v[0], v[1], v[2], v[3], v[4], st);
-    Py_END_ALLOW_THREADS;
-    return PyLong_FromLong(rc);
-}
-
-// (A, Q, w1, w3, inter_size, K, group_size)
-PyObject* deploy_w13(PyObject*, PyObject* const* a, Py_ssize_t n)
-{
-    void *    p[2], *scales[2], *st;
-    uint32_t *qweight[2], *qzeros[2];
-    int       v[3], rc;
-    if (n != 7 || !addresses(a, 2, p) || !triples(a + 2, 2, qweight, qzeros, scales) || !numbers(a + 4, 3, v) || !stream_of(Py_None, &st))
-        Py_RETURN_NONE;
-    Py_BEGIN_ALLOW_THREADS;
-    rc = fn_deploy_w13(static_cast<uint32_t*>(p[0]), p[1], qweight[0], qweight[1], qzeros[0], qzeros[1], scales[0], scales[1], v[0], v[1],
-                       v[2], st);
+    rc = fn_deploy_layer(dst, Q, qweight, qzeros, scales, width, rows, v[0], v[1], st);
     Py_END_ALLOW_THREADS;
     return PyLong_FromLong(rc);
 }
@@ -211,30 +208,29 @@ PyObject* ptr(PyObject*, PyObject* t)
     return PyLong_FromVoidPtr(p);
 }
 
-// (addresses of the six functions above, accessor of the current device, of its current stream, torch.nn.Parameter)
+// (addresses of the five functions above, accessor of the current device, of its current stream, torch.nn.Parameter)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
-    void* f[6];
-    bool  ok = n == 9;
-    for (int i = 0; ok && i < 6; ++i) ok = pointer(a[i], &f[i]);
+    void* f[5];
+    bool  ok = n == 8;
+    for (int i = 0; ok && i < 5; ++i) ok = pointer(a[i], &f[i]);
     if (!ok) {
-        PyErr_SetString(PyExc_TypeError, "bind: six addresses, two accessors and a type");
+        PyErr_SetString(PyExc_TypeError, "bind: five addresses, two accessors and a type");
         return nullptr;
     }
-    fn_gemm        = reinterpret_cast<decltype(fn_gemm)>(f[0]);
-    fn_gemm_static = reinterpret_cast<decltype(fn_gemm_static)>(f[1]);
-    fn_ffn         = reinterpret_cast<decltype(fn_ffn)>(f[2]);
-    fn_convert     = reinterpret_cast<decltype(fn_convert)>(f[3]);
-    fn_deploy_qkv  = reinterpret_cast<decltype(fn_deploy_qkv)>(f[4]);
-    fn_deploy_w13  = reinterpret_cast<decltype(fn_deploy_w13)>(f[5]);
-    for (int i = 6; i < 9; ++i) Py_INCREF(a[i]);
-    get_device = a[6], get_stream = a[7], parameter_type = a[8];
+    fn_gemm         = reinterpret_cast<decltype(fn_gemm)>(f[0]);
+    fn_gemm_static  = reinterpret_cast<decltype(fn_gemm_static)>(f[1]);
+    fn_ffn          = reinterpret_cast<decltype(fn_ffn)>(f[2]);
+    fn_convert      = reinterpret_cast<decltype(fn_convert)>(f[3]);
+    fn_deploy_layer = reinterpret_cast<decltype(fn_deploy_layer)>(f[4]);
+    for (int i = 5; i < 8; ++i) Py_INCREF(a[i]);
+    get_device = a[5], get_stream = a[6], parameter_type = a[7];
     Py_RETURN_NONE;
 }
 
 #define W4A16_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {W4A16_FAST(bind), W4A16_FAST(gemm), W4A16_FAST(gemm_static), W4A16_FAST(ffn), W4A16_FAST(convert),
-                         W4A16_FAST(deploy_qkv), W4A16_FAST(deploy_w13), W4A16_FAST(describe),
+                         W4A16_FAST(deploy_layer), W4A16_FAST(describe),
                          {"ptr", ptr, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

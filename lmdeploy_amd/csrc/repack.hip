@@ -104,7 +104,8 @@ __global__ void __launch_bounds__(kThreads) deploy_q_kernel(uint32_t* __restrict
 // vectors, which lanes exchange through LDS so that a store covers 256 contiguous bytes of four tiles; the (zero, scale) words
 // ride in the same launch.  Bound by HBM: every byte is read and written once.  Stored as the threads held them, sixteen bytes
 // in each of 64 cache lines at a time, the weights kept the L2s busy with requests: Llama-2-70B's four matrices (899 MB moved)
-// 222.6 us, 4.0 TB/s, exchanged first 178, and with non-temporal stores 168.8, 5.3 TB/s (a device copy reaches 5.15).
+// 222.6 us, 4.0 TB/s, exchanged first 178, and with non-temporal stores 168.8, 5.3 TB/s (a device copy reaches 5.15), in one launch
+// 158.2.
 struct TilePair {
     const uint32_t* qw[2];  // the two word columns of the tile
     const uint32_t* qz[2];
@@ -162,17 +163,40 @@ __device__ __forceinline__ void transpose_nibbles(uint32_t (&a)[8])
     }
 }
 
-// Blocks [0, w_blocks) convert weights: 64 word columns (32 tiles) of one row of tiles, wave b the rows 32j + 8b ..
-// Blocks beyond build the Q words of 256 tiles' columns of one quantisation group row each.
-__global__ void __launch_bounds__(kThreads)
-convert_tiles_kernel(uint32_t* __restrict__ dst, uint32_t* __restrict__ Q, const ColumnSource cs, int NT, int G,
-                     int w_across, int w_blocks, int q_across)
+// One launch converts several matrices, each by a run of blocks of its own: those of a decoder layer one by one paid for
+// three more kernel boundaries and ramps (Llama-2-7B's 213 MB: four launches 46.9 us, one 37.5; Llama-2-70B's 899 MB 168.8 and 158.2).
+struct Conversion {
+    ColumnSource cs;
+    uint32_t*    dst;
+    uint32_t*    Q;
+    int          NT;
+    int          w_across, w_blocks, q_across;
+    int          end;  // the first block of the next matrix
+};
+template<int M>
+struct Conversions {
+    Conversion of[M];
+};
+
+// A matrix's first w_blocks blocks convert weights: 64 word columns (32 tiles) of one row of tiles, wave b the rows 32j + 8b ..
+// Those beyond build the Q words of 256 tiles' columns of one quantisation group row each.
+template<int M>
+__global__ void __launch_bounds__(kThreads) convert_tiles_kernel(const Conversions<M> all)
 {
     __shared__ u32x4_t exchange[4][512];  // one part for each wave, which waits for nobody else
     const int          tid = threadIdx.x;
-    if ((int)blockIdx.x < w_blocks) {
-        const int kt   = blockIdx.x / w_across;
-        const int base = (blockIdx.x % w_across) * 64;  // first word column: tile base / 2
+    int                which = 0, block = blockIdx.x;
+#pragma unroll
+    for (int i = 0; i + 1 < M; ++i)
+        if ((int)blockIdx.x >= all.of[i].end) which = i + 1, block = (int)blockIdx.x - all.of[i].end;
+    const Conversion&   of = all.of[which];
+    const ColumnSource& cs = of.cs;
+    uint32_t* const     dst = of.dst;
+    uint32_t* const     Q   = of.Q;
+    const int           NT  = of.NT;
+    if (block < of.w_blocks) {
+        const int kt   = block / of.w_across;
+        const int base = (block % of.w_across) * 64;  // first word column: tile base / 2
         const int lane = tid & 63, b = tid >> 6;
         const int at   = min(base + lane, 2 * NT - 1);  // word column: tile at / 2, word at % 2
         const int nt = at >> 1, h = at & 1;
@@ -206,9 +230,9 @@ convert_tiles_kernel(uint32_t* __restrict__ dst, uint32_t* __restrict__ Q, const
         }
         return;
     }
-    const int blk = blockIdx.x - w_blocks;
-    const int g   = blk / q_across;
-    const int nt  = (blk % q_across) * kThreads + tid;
+    const int blk = block - of.w_blocks;
+    const int g   = blk / of.q_across;
+    const int nt  = (blk % of.q_across) * kThreads + tid;
     if (nt >= NT) return;
     const TilePair t = locate_tile(cs, nt);
     uint32_t       z[2], out[16];
@@ -401,51 +425,104 @@ inline unsigned blocks_for(int64_t n)
 
 }  // namespace
 
-// Q == nullptr: the weights alone
-static hipError_t launch_columns(uint32_t* A_dst, uint32_t* Q_dst, const ColumnSource& cs, int m, int k, int group, hipStream_t st)
+namespace {
+
+// one matrix's conversion: columns gathered as `cs` says, rows of K, quantisation groups; Q == nullptr: the weights alone
+struct Matrix {
+    ColumnSource cs;
+    uint32_t *   A, *Q;
+    int          m, k;
+};
+
+// Whole tiles: no tile straddles two sources or two heads, and every vector access is aligned.  Appends the matrix to a launch of
+// `blocks` blocks so far, false if it (or the launch with it) has to go another way.
+bool as_tiles(const Matrix& x, int group, int64_t& blocks, Conversion& c)
 {
-    const int64_t words = (int64_t)m * k / 8;
-    const int     G     = k / group;
-    if (words == 0) return hipSuccess;
-    // whole tiles: no tile straddles two sources or two heads, and every vector access is aligned
     auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    bool tiles   = aligned(A_dst) && aligned(Q_dst);
+    bool tiles   = aligned(x.A) && aligned(x.Q);
     for (int i = 0; i < 3; ++i)
-        if (cs.width[i] > 0)
-            tiles = tiles && (cs.interleave || cs.width[i] % kTileN == 0) && cs.rotary[i] % kTileN == 0 && aligned(cs.s[i]);
-    const int     NT       = m / kTileN;
-    const int     w_across = (2 * NT + 63) / 64, q_across = (NT + kThreads - 1) / kThreads;
-    const int64_t w_blocks = (int64_t)(k / kGroup) * w_across, blocks = w_blocks + (Q_dst ? (int64_t)G * q_across : 0);
-    if (tiles && blocks < (1ll << 31))
-        return launch_kernel(convert_tiles_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, A_dst, Q_dst, cs, NT, G, w_across,
-                             (int)w_blocks, q_across);
-    hipError_t e = launch_kernel(deploy_weights_kernel, dim3(blocks_for(words)), dim3(kThreads), 0, st, A_dst, cs, m, k);
-    if (Q_dst && e == hipSuccess)
-        e = launch_kernel(deploy_q_kernel, dim3(blocks_for((int64_t)G * m)), dim3(kThreads), 0, st, Q_dst, cs, m, G);
+        if (x.cs.width[i] > 0)
+            tiles = tiles && (x.cs.interleave || x.cs.width[i] % kTileN == 0) && x.cs.rotary[i] % kTileN == 0 && aligned(x.cs.s[i]);
+    const int     NT = x.m / kTileN, w_across = (2 * NT + 63) / 64, q_across = (NT + kThreads - 1) / kThreads;
+    const int64_t w_blocks = (int64_t)(x.k / kGroup) * w_across;
+    blocks += w_blocks + (x.Q ? (int64_t)(x.k / group) * q_across : 0);
+    if (!tiles || blocks >= (1ll << 31)) return false;
+    c = Conversion{x.cs, x.A, x.Q, NT, w_across, (int)w_blocks, q_across, (int)blocks};
+    return true;
+}
+
+template<int M>
+hipError_t launch_matrices(const Matrix (&x)[M], int group, hipStream_t st)
+{
+    Conversions<M> all;
+    int64_t        blocks = 0;
+    bool           tiles  = true;
+    for (int i = 0; i < M; ++i) tiles = tiles && as_tiles(x[i], group, blocks, all.of[i]);
+    if (tiles) return blocks ? launch_kernel(convert_tiles_kernel<M>, dim3((unsigned)blocks), dim3(kThreads), 0, st, all) : hipSuccess;
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < M && e == hipSuccess; ++i) {
+        if constexpr (M > 1) {
+            const Matrix one[1] = {x[i]};
+            e                   = launch_matrices(one, group, st);
+        }
+        else {
+            const int64_t words = (int64_t)x[i].m * x[i].k / 8, entries = (int64_t)(x[i].k / group) * x[i].m;
+            if (words == 0) continue;
+            e = launch_kernel(deploy_weights_kernel, dim3(blocks_for(words)), dim3(kThreads), 0, st, x[i].A, x[i].cs, x[i].m, x[i].k);
+            if (x[i].Q && e == hipSuccess)
+                e = launch_kernel(deploy_q_kernel, dim3(blocks_for(entries)), dim3(kThreads), 0, st, x[i].Q, x[i].cs, x[i].m, x[i].k / group);
+        }
+    }
     return e;
 }
+
+Matrix plain(uint32_t* A_dst, uint32_t* Q_dst, const uint32_t* A_src, const uint16_t* scales, const uint32_t* qzeros, int m, int k)
+{
+    Matrix x{{}, A_dst, Q_dst, m, k};
+    x.cs.qw[0] = A_src, x.cs.qz[0] = qzeros, x.cs.s[0] = scales, x.cs.width[0] = m;
+    return x;
+}
+
+Matrix gathered(uint32_t* A_dst, uint32_t* Q_dst, const uint32_t* const qw[3], const uint32_t* const qz[3], const uint16_t* const s[3],
+                const int width[3], const int rotary[3], int interleave, int k)
+{
+    Matrix x{{}, A_dst, Q_dst, 0, k};
+    for (int i = 0; i < 3; ++i) {
+        x.cs.qw[i] = qw[i], x.cs.qz[i] = qz[i], x.cs.s[i] = s[i];
+        x.cs.width[i] = width[i], x.cs.rotary[i] = rotary[i];
+        x.m += width[i];
+    }
+    x.cs.interleave = interleave;
+    return x;
+}
+
+}  // namespace
 
 hipError_t launch_convert(uint32_t* A_dst, uint32_t* Q_dst, const uint32_t* A_src, const uint16_t* scales,
                           const uint32_t* qzeros, int m, int k, int group, hipStream_t st)
 {
-    ColumnSource cs{};
-    cs.qw[0] = A_src, cs.qz[0] = qzeros, cs.s[0] = scales, cs.width[0] = m;
-    return launch_columns(A_dst, Q_dst, cs, m, k, group, st);
+    const Matrix one[1] = {plain(A_dst, Q_dst, A_src, scales, qzeros, m, k)};
+    return launch_matrices(one, group, st);
 }
 
 hipError_t launch_deploy(uint32_t* A_dst, uint32_t* Q_dst, const uint32_t* const qw[3], const uint32_t* const qz[3],
                          const uint16_t* const s[3], const int width[3], const int rotary[3], int interleave, int k,
                          int group, hipStream_t st)
 {
-    ColumnSource cs{};
-    int          m = 0;
-    for (int i = 0; i < 3; ++i) {
-        cs.qw[i] = qw[i], cs.qz[i] = qz[i], cs.s[i] = s[i];
-        cs.width[i] = width[i], cs.rotary[i] = rotary[i];
-        m += width[i];
-    }
-    cs.interleave = interleave;
-    return launch_columns(A_dst, Q_dst, cs, m, k, group, st);
+    const Matrix one[1] = {gathered(A_dst, Q_dst, qw, qz, s, width, rotary, interleave, k)};
+    return launch_matrices(one, group, st);
+}
+
+hipError_t launch_deploy_layer(uint32_t* const A[4], uint32_t* const Q[4], const uint32_t* const qw[7], const uint32_t* const qz[7],
+                               const uint16_t* const s[7], const int n[7], const int k[4], int size_per_head, int group, hipStream_t st)
+{
+    const uint32_t *const gate_up[3] = {qw[4], qw[5], nullptr}, *const gate_up_z[3] = {qz[4], qz[5], nullptr};
+    const uint16_t* const gate_up_s[3] = {s[4], s[5], nullptr};
+    const int             heads[3] = {size_per_head, size_per_head, 0}, none[3] = {0, 0, 0}, gate_up_n[3] = {n[4], n[5], 0};
+    const Matrix          layer[4] = {gathered(A[0], Q[0], qw, qz, s, n, heads, 0, k[0]), plain(A[1], Q[1], qw[3], s[3], qz[3], n[3], k[1]),
+                                      gathered(A[2], Q[2], gate_up, gate_up_z, gate_up_s, gate_up_n, none, 1, k[2]),
+                                      plain(A[3], Q[3], qw[6], s[6], qz[6], n[6], k[3])};
+    return launch_matrices(layer, group, st);
 }
 
 hipError_t launch_unpack(uint32_t* qweight, uint32_t* qzeros, uint16_t* scales, const uint32_t* A,

@@ -142,6 +142,9 @@ hipError_t launch_convert(uint32_t* A_dst, uint32_t* Q_dst, const uint32_t* A_sr
 hipError_t launch_deploy(uint32_t* A_dst, uint32_t* Q_dst, const uint32_t* const qw[3], const uint32_t* const qz[3],
                          const uint16_t* const s[3], const int width[3], const int rotary[3], int interleave, int k,
                          int group, hipStream_t st);
+// q, k, v, o, gate, up, down in; q|k|v, o, gate|up, down out
+hipError_t launch_deploy_layer(uint32_t* const A[4], uint32_t* const Q[4], const uint32_t* const qw[7], const uint32_t* const qz[7],
+                               const uint16_t* const s[7], const int n[7], const int k[4], int size_per_head, int group, hipStream_t st);
 hipError_t launch_unpack(uint32_t* qweight, uint32_t* qzeros, uint16_t* scales, const uint32_t* A,
                          const uint32_t* Q, int m, int k, int group, hipStream_t st);
 hipError_t launch_dequantize_repacked(uint16_t* W, const uint32_t* A, const uint32_t* Q, int m, int k, int group,

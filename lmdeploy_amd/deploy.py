@@ -7,9 +7,8 @@ loading of `loadWeights` (`src/turbomind/models/llama/LlamaDecoderLayerWeight.cc
 What is kept from the reference: tensor names (`model.layers.{i}.self_attn.q_proj.qweight` ...),
 the result of its deploy steps - q/k rotary re-ordering (`:371-383`, `:633-639`), q|k|v side by side
 (`:251-260`), gate/up columns interleaved (`:641-658`), conversion (`:660-670`) - which the library
-computes per fused tensor in one gather (`w4a16_deploy_qkv`, `w4a16_deploy_w13`), the
-output file names `layers.{i}.attention.w_qkv.{rank}.qweight` / `.scales_zeros` (`:717-757`,
-`:172-192`) with their exact byte sizes (`.qweight` K*N/2, `.scales_zeros` K/128*N*4,
+computes in one gather (`w4a16_deploy_layer`), the output file names
+`layers.{i}.attention.w_qkv.{rank}.qweight` / `.scales_zeros` (`:717-757`, `:172-192`) with their exact byte sizes (`.qweight` K*N/2, `.scales_zeros` K/128*N*4,
 `utils/memory_utils.cu:332-346`), and the `config.ini` keys `weight_type = int4`,
 `group_size = 128` (`:223-224`).
 
@@ -40,24 +39,15 @@ SIZE_PER_HEAD = 128
 def convert_awq_layer(get: Callable[[str], torch.Tensor], i: int, group_size: int = 128) -> Dict[str, torch.Tensor]:
     """The int4 tensors of decoder layer `i` (deploy.py:676-757): `get(name)` returns the
     checkpoint tensor of that name on the GPU, contiguous.  Returns the eight deployable tensors
-    keyed by the reference's parameter names (without the rank infix).  The library builds each fused
-    tensor in one pass from the checkpoint's tensors (`w4a16_deploy_qkv`, `w4a16_deploy_w13`); wo and
-    w2 need only the layout conversion."""
+    keyed by the reference's parameter names (without the rank infix).  The library builds them in one pass
+    over the checkpoint's tensors (`w4a16_deploy_layer`)."""
     def awq(prefix: str):
         return tuple(get(prefix + "." + part) for part in ("qweight", "qzeros", "scales"))
 
-    def plain(prefix: str):
-        qw, qz, s = awq(prefix)
-        A, Q = torch.empty_like(qw), torch.empty_like(s, dtype=torch.int32)   # Q: half2 per (group, feature)
-        tm.convert_s4_k_m8(A, Q, None, qw, s, qz, qw.size(-1) * 8, qw.size(0), group_size)
-        return A, Q
-
     att, mlp = "model.layers.%d.self_attn." % i, "model.layers.%d.mlp." % i
-    made = {"attention.w_qkv": tm.deploy_qkv(awq(att + "q_proj"), awq(att + "k_proj"), awq(att + "v_proj"),
-                                             SIZE_PER_HEAD, group_size),
-            "attention.wo": plain(att + "o_proj"),
-            "feed_forward.w13": tm.deploy_w13(awq(mlp + "gate_proj"), awq(mlp + "up_proj"), group_size),
-            "feed_forward.w2": plain(mlp + "down_proj")}
+    parts = [awq(att + "%s_proj" % name) for name in "qkvo"] + [awq(mlp + "%s_proj" % name) for name in ("gate", "up", "down")]
+    made = dict(zip(("attention.w_qkv", "attention.wo", "feed_forward.w13", "feed_forward.w2"),
+                    tm.deploy_layer(*parts, SIZE_PER_HEAD, group_size)))
     out = {}
     for key, (A, Q) in made.items():
         out["layers.%d.%s.qweight" % (i, key)] = A

@@ -71,11 +71,8 @@ def transpose_qk_s4_k_m8(src, dst, m: int, k: int, size_per_head: int) -> None:
     check(lib.w4a16_transpose_qk_s4_k_m8_hf(_ptr(dst), _ptr(src), m, k, size_per_head, _stream()))
 
 
-def deploy_qkv(q, k, v, size_per_head: int = 128, group_size: int = 128):
-    """The deployable fused q|k|v matrix from the checkpoint's AWQ tensors: q, k, v are
-    (qweight int32 [K, n/8], qzeros int32 [K/g, n/8], scales fp16 [K/g, n]) triples.  Does what
-    deploy_awq does with transpose_qk_s4 / permute, merge_qkv and convert_s4
-    (lmdeploy/serve/turbomind/deploy.py:251-260,371-383,633-639,660-670) in one pass; returns (A, Q)."""
+def _qkv_sizes(q, k, v, group_size: int):
+    """(rows, columns of q, columns of k and of v) of q, k and v that fit together."""
     K = q[0].size(0)
     n_q, n_kv = q[0].size(-1) * 8, k[0].size(-1) * 8
     if v[0].size(-1) * 8 != n_kv or any(t[0].size(0) != K for t in (k, v)):
@@ -84,32 +81,68 @@ def deploy_qkv(q, k, v, size_per_head: int = 128, group_size: int = 128):
         n = qw.size(-1) * 8
         if qz.numel() * 8 != (K // group_size) * n or s.numel() != (K // group_size) * n:
             raise ValueError("qzeros / scales shape does not match qweight")
-    n = n_q + 2 * n_kv
-    A = torch.empty((K, n // 8), dtype=torch.int32, device=q[0].device)
-    Q = torch.empty((K // group_size, n), dtype=torch.int32, device=q[0].device)
-    rc = binding.deploy_qkv(A, Q, q, k, v, n_q, n_kv, K, size_per_head, group_size)
-    if rc is None:
-        arr = lambda i: (ctypes.c_void_p * 3)(*(_ptr(t[i]) for t in (q, k, v)))
-        rc = lib.w4a16_deploy_qkv(_ptr(A), _ptr(Q), arr(0), arr(1), arr(2), n_q, n_kv, K, size_per_head, group_size, _stream())
-    check(rc)
-    return A, Q
+    return K, n_q, n_kv
 
 
-def deploy_w13(w1, w3, group_size: int = 128):
-    """The deployable fused gate|up matrix from the AWQ triples of gate_proj (w1) and up_proj (w3):
-    fuse_w1_w3_s4 + convert_s4 (deploy.py:641-670) in one pass; returns (A, Q)."""
+def _w13_sizes(w1, w3, group_size: int):
+    """(rows, columns of each) of a gate and an up projection that fit together."""
     K, n = w1[0].size(0), w1[0].size(-1) * 8
     for a, b in zip(w1, w3):
         if a.shape != b.shape:
             raise ValueError("w1 and w3 shapes differ")
     if w1[1].numel() * 8 != (K // group_size) * n or w1[2].numel() != (K // group_size) * n:
         raise ValueError("qzeros / scales shape does not match qweight")
-    A = torch.empty((K, 2 * n // 8), dtype=torch.int32, device=w1[0].device)
-    Q = torch.empty((K // group_size, 2 * n), dtype=torch.int32, device=w1[0].device)
-    rc = binding.deploy_w13(A, Q, w1, w3, n, K, group_size)
-    check(lib.w4a16_deploy_w13(_ptr(A), _ptr(Q), _ptr(w1[0]), _ptr(w3[0]), _ptr(w1[1]), _ptr(w3[1]), _ptr(w1[2]),
-                               _ptr(w3[2]), n, K, group_size, _stream()) if rc is None else rc)
+    return K, n
+
+
+def _fused(K: int, n: int, group_size: int, device):
+    return (torch.empty((K, n // 8), dtype=torch.int32, device=device),
+            torch.empty((K // group_size, n), dtype=torch.int32, device=device))
+
+
+def deploy_qkv(q, k, v, size_per_head: int = 128, group_size: int = 128):
+    """The deployable fused q|k|v matrix from the checkpoint's AWQ tensors: q, k, v are
+    (qweight int32 [K, n/8], qzeros int32 [K/g, n/8], scales fp16 [K/g, n]) triples.  Does what
+    deploy_awq does with transpose_qk_s4 / permute, merge_qkv and convert_s4
+    (lmdeploy/serve/turbomind/deploy.py:251-260,371-383,633-639,660-670) in one pass; returns (A, Q)."""
+    K, n_q, n_kv = _qkv_sizes(q, k, v, group_size)
+    A, Q = _fused(K, n_q + 2 * n_kv, group_size, q[0].device)
+    arr = lambda i: (ctypes.c_void_p * 3)(*(_ptr(t[i]) for t in (q, k, v)))
+    check(lib.w4a16_deploy_qkv(_ptr(A), _ptr(Q), arr(0), arr(1), arr(2), n_q, n_kv, K, size_per_head, group_size, _stream()))
     return A, Q
+
+
+def deploy_w13(w1, w3, group_size: int = 128):
+    """The deployable fused gate|up matrix from the AWQ triples of gate_proj (w1) and up_proj (w3):
+    fuse_w1_w3_s4 + convert_s4 (deploy.py:641-670) in one pass; returns (A, Q)."""
+    K, n = _w13_sizes(w1, w3, group_size)
+    A, Q = _fused(K, 2 * n, group_size, w1[0].device)
+    check(lib.w4a16_deploy_w13(_ptr(A), _ptr(Q), _ptr(w1[0]), _ptr(w3[0]), _ptr(w1[1]), _ptr(w3[1]), _ptr(w1[2]),
+                               _ptr(w3[2]), n, K, group_size, _stream()))
+    return A, Q
+
+
+def deploy_layer(q, k, v, o, w1, w3, w2, size_per_head: int = 128, group_size: int = 128):
+    """All matrices of a decoder layer from their AWQ triples in one launch: the pairs (A, Q) of `deploy_qkv` of q, k, v,
+    `convert_s4_k_m8` of o, `deploy_w13` of w1, w3 and `convert_s4_k_m8` of w2."""
+    K, n_q, n_kv = _qkv_sizes(q, k, v, group_size)
+    F, n_f = _w13_sizes(w1, w3, group_size)
+    for qw, qz, s in (o, w2):
+        g, n = qw.size(0) // group_size, qw.size(-1) * 8
+        if s.numel() != g * n or qz.numel() * 8 != g * n:
+            raise ValueError("scales / qzeros / Q shape does not match m, k, group_size")
+    alike = lambda t: (torch.empty_like(t[0]), torch.empty_like(t[2], dtype=torch.int32))   # Q: half2 per (group, feature)
+    made = (_fused(K, n_q + 2 * n_kv, group_size, q[0].device), alike(o), _fused(F, 2 * n_f, group_size, w1[0].device), alike(w2))
+    parts = (q, k, v, o, w1, w3, w2)
+    n = (n_q, n_kv, n_kv, o[0].size(-1) * 8, n_f, n_f, w2[0].size(-1) * 8)
+    rows = (K, o[0].size(0), F, w2[0].size(0))
+    rc = binding.deploy_layer(made, parts, n, rows, size_per_head, group_size)
+    if rc is None:
+        at = lambda of, i: (ctypes.c_void_p * len(of))(*(_ptr(t[i]) for t in of))
+        rc = lib.w4a16_deploy_layer(at(made, 0), at(made, 1), at(parts, 0), at(parts, 1), at(parts, 2), (ctypes.c_int * 7)(*n),
+                                    (ctypes.c_int * 4)(*rows), size_per_head, group_size, _stream())
+    check(rc)
+    return made
 
 
 def dequantize_s4(src, dst) -> None:

@@ -32,6 +32,19 @@ def test_other_forms_are_left_to_the_general_path():
         tm.gemm_static(None, None, None, None, 128, 1, 128, 128, stream=0)
 
 
+def test_validation_of_a_layer():
+    ptrs = lambda n, skip=-1: (ctypes.c_void_p * n)(*[None if i == skip else 0x2000 for i in range(n)])
+    ints = lambda *v: (ctypes.c_int * len(v))(*v)
+    call = lambda A=ptrs(4), Q=ptrs(4), w=ptrs(7), n=(256, 128, 128, 256, 512, 512, 256), k=(256, 256, 256, 512), D=128, g=128: \
+        lib.w4a16_deploy_layer(A, Q, w, ptrs(7), ptrs(7), ints(*n), ints(*k), D, g, None)
+    assert call(g=16) == -1 and call(D=96) == -2 and call(D=3) == -2 and call(D=0) == -2
+    assert call(n=(256, 128, 256, 256, 512, 512, 256)) == -2 and call(n=(256, 128, 128, 256, 512, 504, 256)) == -2
+    assert call(n=(256, 128, 128, 264, 512, 512, 256)) == -2 and call(n=(256, 128, 128, 256, 516, 516, 256)) == -2
+    assert call(k=(256, 200, 256, 512)) == -2 and call(k=(256, -128, 256, 512)) == -4 and call(n=(-256, 128, 128, 256, 512, 512, 256)) == -4
+    assert call(A=None) == -4 and call(A=ptrs(4, 2)) == -4 and call(Q=ptrs(4, 3)) == -4 and call(w=ptrs(7, 5)) == -4
+    assert call(n=(0,) * 7) == 0 and call(k=(0,) * 4) == 0      # nothing to do
+
+
 @pytest.mark.parametrize("count", [0, 1, 5])
 def test_descriptors(count):
     gemms = [(None, None, None, None, 8 * i, -i, i % 3, None, i % 2 == 0) for i in range(count)]
@@ -74,9 +87,8 @@ def test_both_paths_give_the_same():
     tm.convert_s4_k_m8(other(A2), Q2, None, qw, other(s), qz, N, K, g)
     assert torch.equal(A2, A) and torch.equal(Q2, Q)
     plain, mixed = (qw, qz, s), (other(qw), qz, other(s))
-    for made in (tm.deploy_qkv(plain, plain, mixed, 128, g), tm.deploy_w13(plain, list(plain), g)):
-        want = tm.deploy_qkv(plain, plain, plain, 128, g) if made[0].size(-1) == 3 * N // 8 else tm.deploy_w13(plain, plain, g)
-        assert torch.equal(made[0], want[0]) and torch.equal(made[1], want[1])
+    for a, b in zip(tm.deploy_layer(*[plain] * 6, mixed, 128, g), tm.deploy_layer(*[plain] * 7, 128, g)):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
     with pytest.raises(ValueError, match="contiguous"):
         op.Run(out[0], A, X.t(), Q, N, T, K, g)
     with pytest.raises(RuntimeError):  # inside a transform a tensor has no address

@@ -178,3 +178,31 @@ def test_conversion_of_any_number_of_tiles(tiles):
     A_ref, Q_ref = O.convert_s4_k_m8(d["qweight"], d["scales"], d["qzeros"], N, K, G)
     assert np.array_equal(A[:K].cpu().numpy().view(np.uint32).reshape(-1), A_ref) and not A[K:].any()
     assert np.array_equal(Q.cpu().numpy().view(np.uint32), Q_ref)
+
+
+# (hidden, q, kv, inter, head size, group): whole tiles; one tile and a group more than the blocks' shares; a grouped-query layer
+# with a matrix without rows; heads that tiles straddle (every matrix its own launch, a gather per word)
+@pytest.mark.parametrize("h,n_q,n_kv,f,D,g", [(512, 512, 256, 1408, 128, 128), (128, 528, 16, 520, 16, 32), (640, 1024, 128, 0, 128, 64),
+                                              (256, 48, 24, 136, 24, 64)])
+def test_a_layer_in_one_launch_equals_its_matrices_one_by_one(h, n_q, n_kv, f, D, g):
+    import lmdeploy_amd.turbomind as tm
+    rng = np.random.default_rng(h + f)
+    dev = lambda t: tuple(torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)).cuda() for a in t)
+    down = 128 * (f // 128)
+    sizes = ((h, n_q), (h, n_kv), (h, n_kv), (down + 128, h), (h, f), (h, f), (down, h))
+    q, k, v, o, w1, w3, w2 = parts = [dev(_awq(rng, K, N, g)) for K, N in sizes]
+
+    def plain(t):
+        A, Q = torch.empty_like(t[0]), torch.empty_like(t[2], dtype=torch.int32)
+        tm.convert_s4_k_m8(A, Q, None, t[0], t[2], t[1], t[0].size(1) * 8, t[0].size(0), g)
+        return A, Q
+
+    want = tm.deploy_qkv(q, k, v, D, g), plain(o), tm.deploy_w13(w1, w3, g), plain(w2)
+    for given in (parts, [list(t) for t in parts]):
+        got = tm.deploy_layer(*given, D, g)
+        for a, b in zip(got, want):
+            assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    with pytest.raises(ValueError):
+        tm.deploy_layer(q, k, v, (o[0], o[1][:-1], o[2]), w1, w3, w2, D, g)
+    with pytest.raises(tm.W4A16Error):
+        tm.deploy_layer(*parts, 3, g)
