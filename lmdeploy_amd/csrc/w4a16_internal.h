@@ -68,7 +68,7 @@ struct Algo {
     TileConfig   tc;       // tile only
     int          depth;    // K steps come in multiples of this
     int          resident; // workgroups that fit a CU
-    Cost         cost;
+    Cost         cost, few;  // few: up to 128 tokens
 };
 
 // Scratch of the split-K kernels: fp32 partial tiles and arrival counters.  A handle's scratch has
