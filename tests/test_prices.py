@@ -5,7 +5,7 @@ import pytest
 
 from test_choice_per_device import Scratch
 
-BATCH = 4       # w4a16::Family
+STRIP, BATCH = 1, 4       # w4a16::Family
 
 
 def chosen(N, K, T, nq=1):
@@ -19,11 +19,17 @@ def chosen(N, K, T, nq=1):
 
 
 @pytest.mark.parametrize("N,K,T,columns,splits", [
-    (4096, 8192, 9, 16, 1), (4096, 10240, 16, 32, 2), (4096, 20352, 16, 32, 2), (4096, 20480, 16, 64, 4), (2048, 8064, 16, 16, 1),
-    (2048, 8192, 9, 16, 2), (2048, 10240, 9, 32, 4), (5120, 10112, 12, 32, 1), (5120, 10240, 12, 48, 2), (8192, 16256, 16, 32, 1),
+    (4096, 8192, 9, 16, 1), (4096, 10240, 16, 32, 2), (4096, 20352, 16, 32, 2), (4096, 20480, 16, 64, 4), (2048, 7040, 16, 16, 1),
+    (2048, 7168, 9, 16, 2), (2048, 9216, 9, 32, 4), (1024, 4992, 16, 16, 1), (1024, 5120, 9, 16, 4), (1024, 8192, 8, 16, 4), (1536, 12288, 5, 32, 4), (5120, 10112, 12, 32, 1), (5120, 10240, 12, 48, 2), (8192, 16256, 16, 32, 1),
     (8192, 16384, 16, 64, 2), (12288, 28672, 16, 48, 1)])
-def test_a_dozen_tokens_split_deep_matrices(N, K, T, columns, splits):
+def test_up_to_sixteen_tokens_split_deep_matrices(N, K, T, columns, splits):
     assert chosen(N, K, T) == (BATCH, columns, 16, splits)
+
+
+@pytest.mark.parametrize("N,K,T,nq", [(1024, 8064, 8, 1), (1536, 12160, 8, 1), (4096, 28672, 8, 1), (2048, 4096, 5, 2), (512, 4096, 8, 4),
+                                      (1024, 28672, 4, 1)])
+def test_up_to_eight_tokens_stay_with_strips_below_the_line(N, K, T, nq):
+    assert chosen(N, K, T, nq)[0] == STRIP
 
 
 # (the second prices, asked alone, would move each of these to MFMA tiles, which round the weights)
