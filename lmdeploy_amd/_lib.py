@@ -1,9 +1,11 @@
 """ctypes binding of libw4a16.so.  There is no fallback: if the library is missing or lacks a
-symbol, importing fails loudly."""
+symbol, importing fails loudly.  The extension over it (csrc/binding.cpp) only saves host time: where it has not been
+built, every call goes through ctypes."""
 from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from ctypes import (POINTER, Structure, c_char_p, c_double, c_float, c_int, c_longlong, c_size_t, c_ulonglong,
                     c_void_p)
 
@@ -96,9 +98,21 @@ def _load() -> ctypes.CDLL:
 lib = _load()
 
 
+class General:
+    """Stands in for the extension where there is none: each of its functions leaves the call to the general path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def _bind():
     """The calls of a decode step and of a layer's conversion without ctypes (csrc/binding.cpp), through the functions of the library loaded above."""
-    from . import _binding  # ImportError if it has not been built
+    try:
+        from . import _binding
+    except ImportError as e:
+        warnings.warn("lmdeploy_amd._binding cannot be loaded (%s; `python -m lmdeploy_amd.build` makes it): calls go through ctypes, "
+                      "which takes the host longer" % e, RuntimeWarning, stacklevel=2)
+        return General()
     at = lambda fn: ctypes.cast(fn, c_void_p).value
     # torch's own accessors of the current device and of its current stream's handle: torch.cuda.current_stream() wraps
     # the same two in a Stream object, which takes 2.9 us against 0.2 us - more than the whole C call below it

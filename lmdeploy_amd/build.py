@@ -11,6 +11,7 @@ import subprocess
 import sys
 import sysconfig
 from concurrent.futures import ThreadPoolExecutor
+from typing import Optional
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -118,12 +119,23 @@ def build_library(verbose: bool = True) -> str:
     return LIB_PATH
 
 
-def build_binding(verbose: bool = True) -> str:
-    """Compiles csrc/binding.cpp, host code against Python's and torch's headers; it finds the library at run time."""
+def build_binding(verbose: bool = True) -> Optional[str]:
+    """Compiles csrc/binding.cpp, host code against Python's and torch's headers; it finds the library at run time.  Nothing but
+    speed depends on it: without a C++ compiler or those headers it is left out (an older one, which may call the
+    library's functions differently, too), and every call goes through ctypes."""
     import torch
     root = os.path.dirname(torch.__file__)
+    cxx = shutil.which("g++") or shutil.which("c++")
+    headers = [os.path.join(sysconfig.get_paths()["include"], "Python.h"),
+               os.path.join(root, "include", "torch", "csrc", "autograd", "python_variable.h")]
+    missing = ([] if cxx else ["a C++ compiler"]) + [h for h in headers if not os.path.exists(h)]
+    if missing:
+        if os.path.exists(BINDING_PATH):
+            os.remove(BINDING_PATH)
+        print("not built: %s (missing: %s); calls will go through ctypes" % (BINDING_PATH, ", ".join(missing)))
+        return None
     tmp = BINDING_PATH + ".tmp"
-    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden",
+    cmd = [cxx, "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(), "-I", sysconfig.get_paths()["include"],
            "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
            os.path.join(CSRC, "binding.cpp"), "-o", tmp, "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]

@@ -1,6 +1,9 @@
 """The calls that go from Python to the C ABI without ctypes: plain arguments give what the general path gives, and every other
 form is left to that path, with nothing done."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -59,6 +62,50 @@ def test_descriptors(count):
             assert binding.describe(arr, gemms[:-1] + [bad]) is None, bad
 
 
+def test_a_tree_without_the_extension_imports_and_calls():
+    """The library alone is enough: what the extension would take goes through ctypes, and a warning says so."""
+    code = """
+import sys, warnings
+sys.modules["lmdeploy_amd._binding"] = None     # as if it had not been built
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    import lmdeploy_amd.turbomind as tm
+assert ["ctypes" in str(w.message) for w in seen if "lmdeploy_amd._binding" in str(w.message)] == [True], seen
+import ctypes, torch
+for call in (lambda: tm.gemm_static(None, None, None, None, 128, 1, 128, 128, stream=0), lambda: tm.check(tm.lib.w4a16_ffn(*[None] * 9, 128, 128, 1, 128, None))):
+    try:
+        call()
+    except tm.W4A16Error as e:
+        assert e.code == -4 and "null" in str(e)
+    else:
+        raise AssertionError
+try:
+    tm.gemm_static(torch.zeros(2), None, None, None, 128, 1, 128, 128, stream=0)
+except ValueError as e:
+    assert "live on the GPU" in str(e)
+print("fine")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip().endswith("fine"), r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("what", ["compiler", "Python's headers", "torch's headers"])
+def test_a_build_without_what_the_extension_needs_says_so_and_leaves_none(what, monkeypatch, tmp_path, capsys):
+    import lmdeploy_amd.build as build
+    old = tmp_path / "_binding.so"
+    old.write_bytes(b"of another source")
+    monkeypatch.setattr(build, "BINDING_PATH", str(old))
+    if what == "compiler":
+        monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    elif what == "Python's headers":
+        monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    else:
+        monkeypatch.setattr(torch, "__file__", str(tmp_path / "__init__.py"))
+    assert build.build_binding() is None
+    assert not old.exists() and "ctypes" in capsys.readouterr().out
+
+
 @pytest.mark.gpu
 def test_both_paths_give_the_same():
     T, K, N, g = 3, 256, 128, 128
@@ -93,3 +140,36 @@ def test_both_paths_give_the_same():
         op.Run(out[0], A, X.t(), Q, N, T, K, g)
     with pytest.raises(RuntimeError):  # inside a transform a tensor has no address
         torch.vmap(lambda x: op.Run(out[0], A, x, Q, N, T, K, g))(X.expand(2, T, K).contiguous())
+
+
+@pytest.mark.gpu
+def test_every_call_without_the_extension(monkeypatch):
+    from lmdeploy_amd._lib import General
+    T, H, F, g = 3, 256, 512, 128
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    words = lambda *size: torch.randint(-2 ** 31, 2 ** 31, size, dtype=torch.int32, device="cuda", generator=gen)
+    awq = lambda k, n: (words(k, n // 8), words(k // g, n // 8), (torch.rand((k // g, n), device="cuda", generator=gen) * 0.01 + 1e-3).half())
+    parts = [awq(H, H) for _ in range(4)] + [awq(H, F), awq(H, F), awq(F, H)]
+    X, R = torch.randn((2, T, H), device="cuda", generator=gen).half()
+    op = tm.GemmS4F16()
+
+    def everything():
+        new = lambda n: torch.empty((T, n), dtype=torch.float16, device="cuda")
+        (A0, Q0), (A1, Q1), (A2, Q2), (A3, Q3) = made = tm.deploy_layer(*parts, 128, g)
+        A, Q = torch.empty_like(A1), torch.empty_like(Q1)
+        tm.convert_s4_k_m8(A, Q, None, parts[3][0], parts[3][2], parts[3][1], H, H, g)
+        out = [new(3 * H), new(3 * H), new(F), new(H), new(H)]
+        op.Run(out[0], A0, X, Q0, 3 * H, T, H, g)
+        tm.gemm_static(out[1], A0, X, Q0, 3 * H, T, H, g)
+        op.ffn(out[3], out[2], X, A2, Q2, A3, Q3, H, F, T, g, residual=R)
+        op.sequence([(out[4], A1, X, Q1, H, H, op.kFusedAdd, R, True)], T, g)
+        torch.cuda.synchronize()
+        return [t for pair in made for t in pair] + [A, Q] + out
+
+    want = everything()
+    absent = General()
+    monkeypatch.setattr(tm, "binding", absent)
+    for name, of in (("_gemm", "gemm"), ("_gemm_static", "gemm_static"), ("_ffn", "ffn"), ("_describe", "describe"), ("_plain_ptr", "ptr")):
+        monkeypatch.setattr(tm, name, getattr(absent, of))
+    for a, b in zip(want, everything()):
+        assert torch.equal(a, b)
