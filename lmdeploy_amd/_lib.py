@@ -109,6 +109,9 @@ def _bind():
     """The calls of a decode step and of a layer's conversion without ctypes (csrc/binding.cpp), through the functions of the library loaded above."""
     try:
         from . import _binding
+        built_for = getattr(_binding, "torch_version", None)
+        if built_for != torch.__version__:  # (it reads tensors as that torch lays them out)
+            raise ImportError("built for torch %s, this is %s" % (built_for, torch.__version__))
     except ImportError as e:
         warnings.warn("lmdeploy_amd._binding cannot be loaded (%s; `python -m lmdeploy_amd.build` makes it): calls go through ctypes, "
                       "which takes the host longer" % e, RuntimeWarning, stacklevel=2)

@@ -17,7 +17,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libw4a16.so")
-BINDING_PATH = os.path.join(HERE, "_binding.so")
+# (named after the interpreter it is built for: another one does not take it for its own)
+BINDING_PATH = os.path.join(HERE, "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))
+BINDING_UNNAMED = os.path.join(HERE, "_binding.so")  # the name of earlier builds, which every interpreter would load
 
 SOURCES = ["api.cpp", "rounding_domain.cpp", "repack.hip", "static_scratch.hip", "probe.hip", "gemm_decode.hip", "gemm_strip.hip", "gemm_strip_groups.hip",
            "gemm_sequence.hip", "gemm_prefill.hip", "gemm_batch.hip", "gemm_tile_g128.hip", "gemm_tile_g64.hip", "gemm_tile_g32.hip"]
@@ -129,14 +131,15 @@ def build_binding(verbose: bool = True) -> Optional[str]:
     headers = [os.path.join(sysconfig.get_paths()["include"], "Python.h"),
                os.path.join(root, "include", "torch", "csrc", "autograd", "python_variable.h")]
     missing = ([] if cxx else ["a C++ compiler"]) + [h for h in headers if not os.path.exists(h)]
+    for old in (BINDING_UNNAMED, BINDING_PATH) if missing else (BINDING_UNNAMED,):
+        if os.path.exists(old):
+            os.remove(old)
     if missing:
-        if os.path.exists(BINDING_PATH):
-            os.remove(BINDING_PATH)
         print("not built: %s (missing: %s); calls will go through ctypes" % (BINDING_PATH, ", ".join(missing)))
         return None
     tmp = BINDING_PATH + ".tmp"
     cmd = [cxx, "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(), "-I", sysconfig.get_paths()["include"],
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(), "-DW4A16_TORCH=\"%s\"" % torch.__version__, "-I", sysconfig.get_paths()["include"],
            "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
            os.path.join(CSRC, "binding.cpp"), "-o", tmp, "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -236,4 +236,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, methods, n
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__binding() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__binding()
+{
+    PyObject* const m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", W4A16_TORCH) != 0) {  // whose layout of a tensor is compiled in
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -4,6 +4,7 @@ import ctypes
 import os
 import subprocess
 import sys
+import sysconfig
 
 import numpy as np
 import pytest
@@ -88,6 +89,39 @@ print("fine")
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.strip().endswith("fine"), r.stderr[-2000:]
+
+
+def test_an_extension_for_another_torch_is_left_alone():
+    """It reads tensors by the layout that it was compiled with: of another torch it takes no call."""
+    code = """
+import sys, types, warnings
+other = types.ModuleType("lmdeploy_amd._binding")
+other.torch_version, other.bind = "0.0.0", None
+sys.modules["lmdeploy_amd._binding"] = other
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    import lmdeploy_amd
+    lmdeploy_amd._binding = other
+    from lmdeploy_amd import _lib
+assert isinstance(_lib.binding, _lib.General) and any("0.0.0" in str(w.message) for w in seen), seen
+print("fine")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip().endswith("fine"), r.stderr[-2000:]
+
+
+def test_the_extension_is_named_after_its_interpreter(monkeypatch, tmp_path):
+    """Another interpreter does not take it for its own, and one without that name, which it would take, is removed by a build."""
+    import lmdeploy_amd.build as build
+    suffix = sysconfig.get_config_var("EXT_SUFFIX")
+    assert "%d%d" % sys.version_info[:2] in suffix and binding.__file__.endswith(suffix)
+    old = tmp_path / "_binding.so"
+    old.write_bytes(b"of another interpreter")
+    monkeypatch.setattr(build, "BINDING_UNNAMED", str(old))
+    monkeypatch.setattr(build, "BINDING_PATH", str(tmp_path / os.path.basename(build.BINDING_PATH)))
+    assert build.build_binding(verbose=False) == build.BINDING_PATH
+    assert [f.name for f in tmp_path.iterdir()] == ["_binding" + suffix]
 
 
 @pytest.mark.parametrize("what", ["compiler", "Python's headers", "torch's headers"])
