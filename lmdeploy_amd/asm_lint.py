@@ -20,6 +20,10 @@ instruction's result against vector instructions, the compiler normally pads wit
 cannot see into inline assembly.  Compiler-generated accumulator moves (`v_accvgpr_*`) must
 therefore not follow an inline-assembly MFMA that writes the same AGPR within `_MFMA_SETTLE` wait
 states, nor write an AGPR that an inline-assembly MFMA reads within the next two.
+
+Lanes that exchange values through LDS need something between the writes and the reads that the compiler moves neither
+across, also where they belong to one wave, which LDS serves in order: a barrier of the workgroup or of the wave.  No LDS read that the
+compiler generates may follow an LDS write of its own without one.
 """
 from __future__ import annotations
 
@@ -266,6 +270,77 @@ def _m0_hazards(name: str, lines: List[Tuple[int, str]]) -> List[str]:
             for ln, code in writes if borrowed]
 
 
+_LDS_WRITE = re.compile(r"^ds_(?:write|store)")
+_LDS_READ = re.compile(r"^ds_(?:read|load)")
+
+
+def _graph(lines: List[Tuple[int, str]]):
+    """-> blocks of a function, each [label, [(line, code, in_asm)], successors by label, falls through].  A barrier of the wave,
+    which is a comment in the assembly, is the code `wave_barrier`."""
+    blocks, cur, label, in_asm = [], [], "<entry>", False
+    for ln, raw in lines:
+        s = raw.strip()
+        if s.startswith(";;#ASM"):
+            in_asm = s.startswith(";;#ASMSTART")
+            continue
+        m = _LABEL.match(raw)
+        if m:
+            blocks.append([label, cur, [], True])
+            label, cur = m.group(1), []
+            continue
+        code = "wave_barrier" if s.startswith("; wave barrier") else raw.split(";")[0].strip()
+        if not code or code.startswith("."):
+            continue
+        m = _BRANCH.match(code)
+        if m or code.startswith("s_endpgm"):
+            blocks.append([label, cur, [m.group(2)] if m else [], bool(m) and m.group(1) == "cbranch"])
+            label, cur = "<after %d>" % ln, []
+            continue
+        cur.append((ln, code, in_asm))
+    blocks.append([label, cur, [], False])
+    return blocks
+
+
+def _reaches(blocks, start, transfer, merge):
+    """The state at the start of every block that can be reached: `start` at the entry, `transfer(state, instructions)` through
+    a block, `merge` where paths join (it has to be monotone); None where nothing arrives."""
+    index = {b[0]: k for k, b in enumerate(blocks)}
+    entry = [None] * len(blocks)
+    entry[0] = start
+    work = [0]
+    while work:
+        k = work.pop()
+        _, ins, succ, fall = blocks[k]
+        st = transfer(entry[k], ins)
+        for j in [index[s] for s in succ if s in index] + ([k + 1] if fall and k + 1 < len(blocks) else []):
+            new = st if entry[j] is None else merge(entry[j], st)
+            if new != entry[j]:
+                entry[j] = new
+                work.append(j)
+    return entry
+
+
+def _lds_hazards(name: str, lines: List[Tuple[int, str]]) -> List[str]:
+    """LDS reads that can follow an LDS write with no barrier between (both the compiler's own)."""
+    out = []
+
+    def transfer(written, ins, report=False):
+        for ln, code, asm in ins:
+            if code == "wave_barrier" or code.startswith("s_barrier"):
+                written = False
+            elif not asm and _LDS_WRITE.match(code):
+                written = True
+            elif not asm and written and report and _LDS_READ.match(code):
+                out.append("%s: line %d reads LDS after a write with no barrier between: %s" % (name, ln, code))
+        return written
+
+    blocks = _graph(lines)
+    for b, at in zip(blocks, _reaches(blocks, False, transfer, lambda x, y: x or y)):
+        if at is not None:
+            transfer(at, b[1], report=True)
+    return out
+
+
 def lint(asm_text: str, only_if_name_has: str = "kernel") -> List[str]:
     """Returns one message per violation (empty list: clean)."""
     out: List[str] = []
@@ -285,6 +360,7 @@ def lint(asm_text: str, only_if_name_has: str = "kernel") -> List[str]:
     for name, lines in funcs:
         out.extend(_mfma_hazards(name, lines))
         out.extend(_m0_hazards(name, lines))
+        out.extend(_lds_hazards(name, lines))
         blocks = _parse(lines)
         index = {b[0]: k for k, b in enumerate(blocks)}
         entry: List[Dict[int, int]] = [None] * len(blocks)  # type: ignore

@@ -39,8 +39,9 @@ def _hipcc() -> str:
 # The GEMM kernels wait for their software-pipelined loads by count.  A register spill would put
 # scratch stores among those loads, and stores complete out of order with loads, so a spilling
 # GEMM kernel is a wrong kernel: the build refuses it.
-NO_SCRATCH = ("gemm_decode.hip", "gemm_strip.hip", "gemm_strip_groups.hip",
-           "gemm_sequence.hip", "gemm_prefill.hip", "gemm_batch.hip",    "gemm_tile_g128.hip", "gemm_tile_g64.hip", "gemm_tile_g32.hip")
+NO_SCRATCH = ("gemm_decode.hip", "gemm_strip.hip", "gemm_strip_groups.hip", "gemm_sequence.hip", "gemm_prefill.hip", "gemm_batch.hip",
+              "gemm_tile_g128.hip", "gemm_tile_g64.hip", "gemm_tile_g32.hip")
+LINTED = NO_SCRATCH + ("repack.hip",)  # checked by asm_lint
 
 
 def _check_no_scratch(src: str, remarks: str) -> None:
@@ -66,9 +67,9 @@ def _check_no_scratch(src: str, remarks: str) -> None:
                                    "parking VGPRs in AGPRs" % (src, name, agprs, allowed))
 
 
-def _check_inflight(src: str, obj_dir: str) -> None:
-    """Second pass over the same source to assembly text, checked by asm_lint: no compiler-generated
-    instruction may touch a register whose inline-assembly load can still be in flight."""
+def _check_assembly(src: str, obj_dir: str) -> None:
+    """Second pass over the same source to assembly text, checked by asm_lint (no compiler-generated
+    instruction may touch a register whose inline-assembly load can still be in flight, and the like)."""
     try:
         from .asm_lint import lint
     except ImportError:  # run as a script
@@ -82,7 +83,7 @@ def _check_inflight(src: str, obj_dir: str) -> None:
         problems = lint(f.read())
     os.remove(asm)
     if problems:
-        raise RuntimeError("%s: %d uses of registers with a load in flight, e.g.\n%s"
+        raise RuntimeError("%s: asm_lint rejects the assembly in %d places, e.g.\n%s"
                            % (src, len(problems), "\n".join(problems[:5])))
 
 
@@ -99,7 +100,8 @@ def _compile(src: str, obj_dir: str) -> str:
         raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, r.stdout, r.stderr))
     if src in NO_SCRATCH:
         _check_no_scratch(src, r.stderr)
-        _check_inflight(src, obj_dir)
+    if src in LINTED:
+        _check_assembly(src, obj_dir)
     return obj
 
 

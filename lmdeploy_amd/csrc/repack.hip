@@ -222,6 +222,7 @@ __global__ void __launch_bounds__(kThreads) convert_tiles_kernel(const Conversio
                 const int col = row_of_nibble(q);
                 mine[tl * 16 + ((t.turn ? 2 * col + h : 8 * h + col) ^ g(tl))] = u32x4_t{in[0][q], in[1][q], in[2][q], in[3][q]};
             }
+        wave_exchange();
         u32x4_t* const out = reinterpret_cast<u32x4_t*>(dst) + ((int64_t)kt * NT + (base >> 1)) * 64 + b * 16 + (lane & 15);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {

@@ -296,10 +296,11 @@ __device__ __forceinline__ void strip_body(const StripParams& p, int col0, u32x4
         else {
 #pragma unroll
             for (int i = 0; i < NXR; ++i) xw[xw_at[i]] = s.x[i];
+            wave_exchange();
 #pragma unroll
             for (int h = 0; h < H; ++h)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) xf[h][j] = __builtin_bit_cast(half8_t, xw[xr_at[h][j]]);  // same wave: LDS keeps the order
+                for (int j = 0; j < 4; ++j) xf[h][j] = __builtin_bit_cast(half8_t, xw[xr_at[h][j]]);
         }
         constexpr int U  = 2;
         constexpr int JN = 4 / NQ;  // k32 chunks per quantisation group

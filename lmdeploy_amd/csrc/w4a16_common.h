@@ -157,6 +157,15 @@ __device__ __forceinline__ void spread_q(uint32_t x, uint32_t* q)
     }
 }
 
+// Between what the lanes of a wave write to LDS and what other lanes of the same wave read of it.  LDS serves a wave in order, so it
+// is no instruction; it keeps the compiler, which sees one thread's accesses to different places, from swapping them.
+__device__ __forceinline__ void wave_exchange()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // n / d for n below some bound: d == 1 has the reciprocal 0, the others floor(2^32 / d) + 1 (exact while n d < 2^32, Granlund
 // and Montgomery), or 1 where the bound does not allow that and n is divided by d.
 inline uint32_t reciprocal(uint64_t bound, uint32_t d)

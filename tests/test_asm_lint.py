@@ -106,3 +106,21 @@ def test_m0_written_by_the_compiler_where_loads_rely_on_it_is_reported():
     assert lint(HEAD + put + dma + "\ts_cmp_eq_u32 m0, s9\n" + dma + TAIL) == []
     msgs = lint(HEAD + put + dma + other + dma + TAIL)
     assert len(msgs) == 1 and "writes M0" in msgs[0]
+
+
+def test_lds_exchanges_need_a_barrier():
+    put, get = "\tds_write_b128 v2, v[4:7]\n", "\tds_read_b128 v[8:11], v3\n"
+    for between in ("\t; wave barrier\n", "\ts_barrier\n"):
+        assert lint(HEAD + get + put + between + get + TAIL) == []
+        # (a barrier on one of two ways is none)
+        assert len(lint(HEAD + put + "\ts_cbranch_scc1 .LBB0_1\n" + between + ".LBB0_1:\n" + get + TAIL)) == 1
+    msgs = lint(HEAD + put + get + TAIL)
+    assert len(msgs) == 1 and "no barrier between" in msgs[0]
+    # across the back edge of a loop
+    assert len(lint(HEAD + ".LBB0_1:\n" + get + put + "\ts_cbranch_scc1 .LBB0_1\n" + TAIL)) == 1
+    assert lint(HEAD + ".LBB0_1:\n\t; wave barrier\n" + get + put + "\ts_cbranch_scc1 .LBB0_1\n" + TAIL) == []
+
+
+def test_the_conversion_is_checked():
+    from lmdeploy_amd import build
+    assert "repack.hip" in build.LINTED
