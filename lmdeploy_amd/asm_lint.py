@@ -24,6 +24,10 @@ states, nor write an AGPR that an inline-assembly MFMA reads within the next two
 Lanes that exchange values through LDS need something between the writes and the reads that the compiler moves neither
 across, also where they belong to one wave, which LDS serves in order: a barrier of the workgroup or of the wave.  No LDS read that the
 compiler generates may follow an LDS write of its own without one.
+
+Assembly that masks its loads and then sets EXEC to all ones, instead of what it found there, may only stand where every
+lane is active: elsewhere it would switch lanes on in the middle of a branch that they did not take.  Kernels start with all
+lanes (their workgroups are whole waves); from there the pass follows EXEC and the scalar registers that hold a copy of it.
 """
 from __future__ import annotations
 
@@ -303,7 +307,7 @@ def _graph(lines: List[Tuple[int, str]]):
 
 def _reaches(blocks, start, transfer, merge):
     """The state at the start of every block that can be reached: `start` at the entry, `transfer(state, instructions)` through
-    a block, `merge` where paths join (it has to be monotone); None where nothing arrives."""
+    a block, `merge(state, state, block)` where paths join (blocks count from -1 down; it has to be monotone); None where nothing arrives."""
     index = {b[0]: k for k, b in enumerate(blocks)}
     entry = [None] * len(blocks)
     entry[0] = start
@@ -313,7 +317,7 @@ def _reaches(blocks, start, transfer, merge):
         _, ins, succ, fall = blocks[k]
         st = transfer(entry[k], ins)
         for j in [index[s] for s in succ if s in index] + ([k + 1] if fall and k + 1 < len(blocks) else []):
-            new = st if entry[j] is None else merge(entry[j], st)
+            new = st if entry[j] is None else merge(entry[j], st, -1 - j)
             if new != entry[j]:
                 entry[j] = new
                 work.append(j)
@@ -335,9 +339,151 @@ def _lds_hazards(name: str, lines: List[Tuple[int, str]]) -> List[str]:
         return written
 
     blocks = _graph(lines)
-    for b, at in zip(blocks, _reaches(blocks, False, transfer, lambda x, y: x or y)):
+    for b, at in zip(blocks, _reaches(blocks, False, transfer, lambda x, y, _: x or y)):
         if at is not None:
             transfer(at, b[1], report=True)
+    return out
+
+
+_SREGS = re.compile(r"s(?:\[(\d+):(\d+)\]|(\d+))")
+_SECOND_RESULT = re.compile(r"v_(?:\w+_co_|div_scale|mad_[ui]64)")
+_NO_LANE = ("part", (None,))
+_NO_RESULT = ("s_cmp", "s_bitcmp", "s_wait", "s_setprio", "s_barrier", "s_nop", "global_", "buffer_", "flat_", "ds_", "wave_barrier")
+
+
+def _common(x, y):
+    return x[:next((k for k, (p, q) in enumerate(zip(x, y)) if p != q), min(len(x), len(y)))]
+
+
+def _within(v):
+    """The narrowings that lead to a mask which holds what a register holds; None: not known."""
+    return None if v is None or v[0] == "rest" else v[1]
+
+
+def _exec_transfer(state, ins, report=None):
+    """What is known of EXEC: the narrowings, by line, that lead from all lanes (none: all of them) to a mask that holds it.
+    state: (EXEC's, ((n, what s[n:n+1] or vcc holds), ...)); a register holds ("mask", narrowings), a part of one ("part",
+    narrowings), no lane ("part", (None,)), or ("rest", narrowings, wider), what the first lacks of the second as long as EXEC is the first."""
+    now, held = state[0], dict(state[1])
+
+    def narrowed(base, ln):
+        """A new mask inside `base`; nothing that was said of an earlier one of this line holds any more."""
+        for n in [n for n, v in held.items() if ln in v[1]]:
+            del held[n]
+        return (base[:base.index(ln)] if ln in base else base) + (ln,)
+
+    def joined(v, ln):
+        """EXEC and what a register holds, together."""
+        if v is None:
+            return narrowed((), ln)
+        if v[0] == "rest":
+            return v[2] if v[1] == now else narrowed((), ln)
+        if v == _NO_LANE or v[0] == "mask" and now[:len(v[1])] == v[1]:
+            return v[1] if v != _NO_LANE else now
+        return narrowed(_common(now, v[1]), ln)
+
+    for ln, code, asm in ins:
+        op, _, rest = code.partition(" ")
+        if op.startswith(_NO_RESULT):
+            continue
+        args = [a.strip() for a in rest.split(",")]
+        if asm and args[0] == "exec":  # the mask of the statement's loads, which ends it with all ones
+            if args[1] == "-1":
+                if now and report is not None:
+                    report(ln, code)
+                now = ()
+            continue
+        m = [_SREGS.fullmatch(a) for a in args]
+        reg = [a if a == "vcc" else int(x.group(1)) if x and x.group(1) else None for a, x in zip(args, m)]
+        fixed = {"exec": ("mask", now), "-1": ("mask", ()), "0": _NO_LANE}
+        value = [fixed.get(a, held.get(n)) for a, n in zip(args, reg)]
+        was, new, also = now, None, None
+        if "saveexec" in op:
+            new, v = ("mask", now), value[1]
+            if op == "s_and_saveexec_b64":
+                now = narrowed(now, ln)
+            elif op == "s_or_saveexec_b64":
+                now = joined(v, ln)
+            elif op == "s_andn2_saveexec_b64" and v is not None and v[0] == "rest" and v[1] == now:  # the other side of a branch
+                now = narrowed(v[2], ln)
+                new = ("rest", now, v[2])
+            else:
+                now = narrowed((), ln)
+            if new[0] == "mask" and ln in new[1]:
+                new = None
+        elif args[0] == "exec":
+            v = value[2] if len(value) > 2 and args[1] == "exec" else None
+            if op == "s_mov_b64" and value[1] is not None and value[1][0] == "mask":
+                now = value[1][1]
+            elif op == "s_or_b64":
+                now = joined(v, ln)
+            elif op == "s_xor_b64" and v is not None and v[0] == "mask" and v[1][:len(now)] == now and v[1] != now:
+                now = narrowed(now, ln)
+                also = (reg[2], ("rest", now, was))
+            else:
+                now = narrowed(now if op in ("s_and_b64", "s_andn2_b64") and args[1] == "exec" else (), ln)
+        elif args[0].startswith("exec"):
+            now = narrowed((), ln)
+        elif op == "s_mov_b64":
+            new = value[1]
+        elif op == "s_xor_b64" and args[1] == "exec" and value[2] is not None and value[2][0] == "mask" and now[:len(value[2][1])] == value[2][1]:
+            new = ("rest", now, value[2][1])
+        elif op in ("s_and_b64", "s_andn2_b64", "s_or_b64"):
+            x, y = map(_within, value[1:3])
+            if op == "s_andn2_b64":
+                part = x
+            elif op == "s_and_b64":
+                part = x if y is None or x is not None and len(x) > len(y) else y
+            else:
+                part = y if x == _NO_LANE[1] else x if y == _NO_LANE[1] else None if x is None or y is None else _common(x, y)
+            new = ("part", part) if part is not None else None
+        elif op.startswith("v_cmpx_"):
+            now = narrowed(now, ln)
+        elif op.startswith("v_cmp_"):
+            new = ("part", now)
+            if op.endswith("_e32"):
+                reg[0] = "vcc"
+        written = m[:2] if _SECOND_RESULT.match(op) else m[:1]
+        for x in written:
+            if x:
+                lo, hi = int(x.group(1) or x.group(3)), int(x.group(2) or x.group(3))
+                for n in [n for n in held if n != "vcc" and n <= hi and n + 1 >= lo]:
+                    del held[n]
+        if any(a.startswith("vcc") for a in args[:2]):
+            held.pop("vcc", None)
+        for n, v in ((reg[0], new), also or (None, None)):
+            if n is not None and v is not None and v != ("part", ()):
+                held[n] = v
+    return now, tuple(sorted(held.items(), key=str))
+
+
+def _exec_merge(x, y, block):
+    now = x[0]
+    if x[0] != y[0]:
+        now = _common(*(z[0][:z[0].index(block)] if block in z[0] else z[0] for z in (x, y))) + (block,)
+    held, other = [], dict(y[1])
+    for n, v in x[1]:
+        w = other.get(n)
+        if w != v:
+            p, q = _within(v), _within(w)
+            part = q if p == _NO_LANE[1] else p if q == _NO_LANE[1] else None if p is None or q is None else _common(p, q)
+            v = ("part", part) if part else None
+        if v is not None and block not in v[1]:
+            held.append((n, v))
+    return now, tuple(held)
+
+
+def _exec_hazards(name: str, lines: List[Tuple[int, str]]) -> List[str]:
+    """Assembly that sets EXEC to all ones where a lane may be switched off."""
+    out: List[str] = []
+    blocks = _graph(lines)
+    if not any(asm and code.replace(" ", "") == "s_mov_b64exec,-1" for b in blocks for _, code, asm in b[1]):
+        return out
+    states = _reaches(blocks, ((), ()), _exec_transfer, _exec_merge)
+    for b, at in zip(blocks, states):
+        if at is not None:
+            _exec_transfer(at, b[1], lambda ln, code: out.append(
+                "%s: line %d switches every lane on where some may be off: %s" % (name, ln, code)))
     return out
 
 
@@ -361,6 +507,7 @@ def lint(asm_text: str, only_if_name_has: str = "kernel") -> List[str]:
         out.extend(_mfma_hazards(name, lines))
         out.extend(_m0_hazards(name, lines))
         out.extend(_lds_hazards(name, lines))
+        out.extend(_exec_hazards(name, lines))
         blocks = _parse(lines)
         index = {b[0]: k for k, b in enumerate(blocks)}
         entry: List[Dict[int, int]] = [None] * len(blocks)  # type: ignore

@@ -74,7 +74,7 @@ constexpr int kEpiRuntime = 3;  // template value: take the epilogue from StripP
 // Loads of the software pipeline: issued from inline assembly, in place ("+v"), with a scalar
 // base, a per-lane 32-bit offset and an immediate, and waited for by count (the compiler would
 // drain every load in flight at the loop header).  They run under an EXEC mask of all lanes or none
-// (every lane is active around them): with none the instructions still issue and still count in vmcnt, but touch
+// (every lane is active around them, which asm_lint.py checks): with none the instructions still issue and still count in vmcnt, but touch
 // neither memory nor their destination, which lets the last trips of a loop skip their refills without
 // a branch - the number of loads in flight stays a compile-time constant.  Up to four loads share one change of the mask:
 // the scalar instructions between the loads of all waves of a SIMD add up.

@@ -1,5 +1,7 @@
 """The build-time assembly check must catch a register that is touched while an inline-assembly
 load into it is still in flight, and must accept the same code once a counted wait covers it."""
+import pytest
+
 from lmdeploy_amd.asm_lint import lint
 
 HEAD = "_ZN5w4a164test_kernelEv:\n"
@@ -124,3 +126,34 @@ def test_lds_exchanges_need_a_barrier():
 def test_the_conversion_is_checked():
     from lmdeploy_amd import build
     assert "repack.hip" in build.LINTED
+
+
+MASKED = "\t;;#ASMSTART\n\ts_mov_b64 exec, s[40:41]\n\tglobal_load_dword v0, v40, s[2:3]\n\ts_mov_b64 exec, -1\n\t;;#ASMEND\n"
+BRANCH = "\ts_and_saveexec_b64 s[10:11], vcc\n\ts_cbranch_execz .LBB0_1\n%s.LBB0_1:\n\ts_or_b64 exec, exec, s[10:11]\n"
+BOTH = ("\ts_and_saveexec_b64 s[10:11], vcc\n\ts_xor_b64 s[10:11], exec, s[10:11]\n\tv_mov_b32_e32 v30, 0\n"
+        "\ts_andn2_saveexec_b64 s[10:11], s[10:11]\n\ts_cbranch_execz .LBB0_1\n%s.LBB0_1:\n\ts_or_b64 exec, exec, s[10:11]\n")
+LOOP = ("\ts_mov_b64 s[20:21], 0\n.LBB0_7:\n%s\tv_cmp_gt_u32_e32 vcc, v30, v31\n\ts_or_b64 s[20:21], vcc, s[20:21]\n"
+        "\ts_andn2_b64 exec, exec, s[20:21]\n\ts_cbranch_execnz .LBB0_7\n\ts_or_b64 exec, exec, s[20:21]\n")
+INNER = "\ts_and_saveexec_b64 s[12:13], s[14:15]\n\tv_mov_b32_e32 v30, 0\n\ts_or_b64 exec, exec, s[12:13]\n"
+
+
+@pytest.mark.parametrize("body", [MASKED, MASKED + MASKED, BRANCH % "" + MASKED, BRANCH % INNER + MASKED, BOTH % INNER + MASKED, BRANCH % LOOP % "" + MASKED,
+                                  "\ts_mov_b64 s[6:7], exec\n\ts_and_b64 exec, exec, vcc\n\ts_mov_b64 exec, s[6:7]\n" + MASKED,
+                                  ".LBB0_2:\n" + BRANCH % INNER + MASKED + "\ts_cbranch_scc1 .LBB0_2\n"])
+def test_masked_loads_where_every_lane_is_active(body):
+    assert lint(HEAD + body + TAIL) == []
+
+
+@pytest.mark.parametrize("body", [
+    BRANCH % MASKED, BOTH % MASKED, BRANCH % (INNER + MASKED), BRANCH % LOOP % MASKED,
+    "\ts_and_b64 exec, exec, vcc\n" + MASKED,
+    "\ts_mov_b64 exec, s[6:7]\n" + MASKED,
+    "\ts_mov_b32 exec_lo, s6\n" + MASKED,
+    BRANCH % "\ts_mov_b32 s11, 0\n" + MASKED,                                  # the saved mask was written over
+    BRANCH % "\tv_add_co_u32_e64 v30, s[10:11], v30, v31\n" + MASKED,
+    "\ts_and_saveexec_b64 s[10:11], vcc\n\ts_cbranch_scc1 .LBB0_1\n\ts_or_b64 exec, exec, s[10:11]\n.LBB0_1:\n" + MASKED,   # restored on one way
+    ".LBB0_2:\n" + MASKED + "\ts_and_b64 exec, exec, vcc\n\ts_cbranch_execnz .LBB0_2\n",                                   # around the back edge
+    LOOP % ("\ts_and_saveexec_b64 s[12:13], vcc\n\ts_xor_b64 s[16:17], exec, s[12:13]\n") + "\ts_or_b64 exec, exec, s[16:17]\n" + MASKED])
+def test_masked_loads_where_a_lane_may_be_off_are_reported(body):
+    msgs = lint(HEAD + body + TAIL)
+    assert len(msgs) == 1 and "switches every lane on" in msgs[0]
