@@ -11,6 +11,8 @@
 // partial strips are added in LDS in slice order.
 #pragma once
 
+#include <stddef.h>
+
 #include "pipeline.h"
 
 namespace w4a16 {
@@ -44,10 +46,21 @@ struct StripParams {
 // microseconds after its launch, and everything in front of the first load counts in full: with this, addresses that advance
 // instead of being multiplied out for every group, and one change of the mask for up to four loads, 4096 x 4096 at one token
 // went from 4.43 to 4.10 us, 4096 x 12288 7.33 -> 6.95, 4096 x 22016 11.42 -> 10.95, 11008 x 4096 7.05 -> 6.62 (cold weights).
-#define STRIP_ARGS                                                                                                     \
-    const u32x4_t *A, const uint16_t *X, const uint32_t *Q, int N, int T, int K, int rem, int passes, uint32_t how,    \
-        uint16_t *C, const uint16_t *Rsd, unsigned long long *clk
-#define STRIP_ARG_NAMES A, X, Q, N, T, K, rem, passes, how, C, Rsd, clk
+// One list, from which their parameters, the parameters' names and their places in memory come.
+#define STRIP_LIST(EACH, LAST)                                                                                         \
+    EACH(const u32x4_t*, A) EACH(const uint16_t*, X) EACH(const uint32_t*, Q) EACH(int, N) EACH(int, T) EACH(int, K)   \
+    EACH(int, rem) EACH(int, passes) EACH(uint32_t, how) EACH(uint16_t*, C) EACH(const uint16_t*, Rsd)                 \
+    LAST(unsigned long long*, clk)
+#define STRIP_PARAM(type, name) type name,
+#define STRIP_LAST_PARAM(type, name) type name
+#define STRIP_NAME(type, name) name,
+#define STRIP_LAST_NAME(type, name) name
+#define STRIP_FIELD(type, name) type name;
+#define STRIP_ARGS STRIP_LIST(STRIP_PARAM, STRIP_LAST_PARAM)
+#define STRIP_ARG_NAMES STRIP_LIST(STRIP_NAME, STRIP_LAST_NAME)
+struct StripMemory {  // (kernel arguments lie in memory as the members of a struct do)
+    STRIP_LIST(STRIP_FIELD, STRIP_FIELD)
+};
 // `how`: workgroups side by side (16 bits, read where they take several strips: one for each CU then), width of a narrow strip (8), epilogue (2), and whether the clock is recorded
 constexpr uint32_t kHowClock = 1u << 31;
 __device__ __forceinline__ StripParams strip_params(STRIP_ARGS)
@@ -66,7 +79,7 @@ __device__ __forceinline__ unsigned long long* strip_clock()
     typedef __attribute__((address_space(1))) unsigned long long* counters;
     auto args = (__attribute__((address_space(4))) const char*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(args));
-    return (unsigned long long*)*(__attribute__((address_space(4))) const counters*)(args + 64);
+    return (unsigned long long*)*(__attribute__((address_space(4))) const counters*)(args + offsetof(StripMemory, clk));
 }
 
 constexpr int kEpiRuntime = 3;  // template value: take the epilogue from StripParams
