@@ -152,7 +152,7 @@ bool triples(PyObject* const* t, int count, uint32_t** qweight, uint32_t** qzero
 // (4 pairs (A, Q), 7 triples (qweight, qzeros, scales), 7 widths, 4 numbers of rows, size_per_head, group_size), tuples all of them
 PyObject* deploy_layer(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
-    void *    Q[4], *scales[7], *p[3], *st;
+    void *    Q[4], *scales[7], *p[2], *st;
     uint32_t *dst[4], *qweight[7], *qzeros[7];
     int       width[7], rows[4], v[2], rc;
     auto      tuple = [](PyObject* o, Py_ssize_t size) { return PyTuple_CheckExact(o) && PyTuple_GET_SIZE(o) == size; };
@@ -162,11 +162,7 @@ PyObject* deploy_layer(PyObject*, PyObject* const* a, Py_ssize_t n)
         ok                = tuple(t, 2) && addresses(PySequence_Fast_ITEMS(t), 2, p);
         if (ok) dst[i] = static_cast<uint32_t*>(p[0]), Q[i] = p[1];
     }
-    for (int i = 0; ok && i < 7; ++i) {
-        PyObject* const t = PyTuple_GET_ITEM(a[1], i);
-        ok                = tuple(t, 3) && addresses(PySequence_Fast_ITEMS(t), 3, p);
-        if (ok) qweight[i] = static_cast<uint32_t*>(p[0]), qzeros[i] = static_cast<uint32_t*>(p[1]), scales[i] = p[2];
-    }
+    ok = ok && triples(PySequence_Fast_ITEMS(a[1]), 7, qweight, qzeros, scales);
     if (!ok || !numbers(PySequence_Fast_ITEMS(a[2]), 7, width) || !numbers(PySequence_Fast_ITEMS(a[3]), 4, rows) || !numbers(a + 4, 2, v) ||
         !stream_of(Py_None, &st))
         Py_RETURN_NONE;
