@@ -298,7 +298,7 @@ batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int 
         __syncthreads();
         int* const last_flag = reinterpret_cast<int*>(smem);
         if (tid == 0) {
-            const bool last = arrive_last(counters + tile, (int)splits, epoch);
+            const bool last = arrive_last(counters, tile, (int)splits, epoch);
             *last_flag = last;
         }
         __syncthreads();

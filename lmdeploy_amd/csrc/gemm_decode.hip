@@ -318,7 +318,7 @@ decode_kernel(const DecodeParams p)
         }
         __syncthreads();
         if (tid == 0) {
-            const bool last = arrive_last(p.cnt + blockIdx.z * gridDim.x + blockIdx.x, p.SK, p.epoch);
+            const bool last = arrive_last(p.cnt, (int)(blockIdx.z * gridDim.x + blockIdx.x), p.SK, p.epoch);
             last_flag = last;
         }
         __syncthreads();

@@ -385,7 +385,7 @@ prefill_kernel(const u32x4_t* __restrict__ A, const uint16_t* __restrict__ X, co
         __syncthreads();                // ... and every wave is done with the activation tiles in LDS
         int* const last_flag = reinterpret_cast<int*>(xs);
         if (tid == 0) {
-            const bool last = arrive_last(cnt + id, splits, epoch);
+            const bool last = arrive_last(cnt, id, splits, epoch);
             *last_flag = last;
         }
         __syncthreads();

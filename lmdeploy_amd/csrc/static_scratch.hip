@@ -16,12 +16,11 @@ namespace w4a16 {
 
 namespace {
 
-constexpr size_t kCounterBytes = 2 * kStaticCounters * sizeof(int);
+constexpr size_t kCounterBytes = 4 * kStaticCounters * sizeof(int);
 constexpr size_t kStaticBytes  = kCounterBytes + kStaticWorkspaceBytes;
 constexpr int    kMaxDevices   = 64;
 
-// [arrival counters: kStaticCounters ints][the second ones, for counts that did not start from zero (arrive_last): as many]
-// [fp32 partial tiles: kStaticWorkspaceBytes]
+// [arrival counters, in three parts (kStaticCounters)][fp32 partial tiles: kStaticWorkspaceBytes]
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];
 
 std::mutex     g_mutex;
@@ -82,7 +81,8 @@ hipError_t prepare_static_counters(Scratch* sc, int n, hipStream_t st)
     if (e != hipSuccess) return e;
     if (cs == hipStreamCaptureStatusNone) return hipSuccess;
     sc->epoch = 0;
-    n         = std::min(n, sc->cnt_len);
+    sc->cnt += kStaticRecorded;
+    n = std::min(n, sc->cnt_len);
     return launch_kernel(fill_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, st, sc->cnt, n);
 }
 

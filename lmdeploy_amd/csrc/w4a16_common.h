@@ -211,34 +211,39 @@ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_t, int tiles_n
 // Split K: a workgroup announces that its partial tile is complete; true for the last of `splits`, which leaves the counter
 // at zero for the next launch.  epoch 0: the counters belong to a handle, which nobody else touches, or were cleared right before
 // this launch.  Otherwise they are shared by every caller on the GPU, and launches that overlapped against the rules may have left
-// anything in them.  Every arrival then adds one and the launch's epoch above it: the j-th to arrive at a counter that started
-// from zero finds j times that, and no other start (but one that is as old as the epochs' period) gives any of them the like.  Where one does not, all of them do not, and they
-// count again on a second counter, whose words say by their tag whose counts they hold; the last one clears both, so
-// that one misuse does not spoil the launches after it and none of them has to be preceded by one that clears the counters.
-// (Tagged words and their exchange loop alone, a load and up to `splits` contended exchanges, made 8192 x 1024 at 16 tokens,
-// split in four, 7.7 us a call; one addition: 5.7.)
-__device__ __forceinline__ bool arrive_last(int* counter, int splits, int epoch)
+// anything in them.  Every arrival then adds one, and the launch's epoch in the upper half of the word: what d arrivals of other
+// launches left is taken for this launch's own only if their epochs add up to d times its own.  Those of one launch do so when
+// the epochs have come round (2^19 - 1 launches), those of several also if one of them has a higher epoch than this launch and their mean is
+// its own.  The sum is exact: d below the splits, at most 4095, and 19 bits of epoch.  Where the count did not start from zero, no
+// arrival of the launch finds what it should, and they count again on a second counter, whose words say by their tag whose
+// counts they hold; the last one clears both, so that one misuse does not spoil the launches after it and none of them has to be
+// preceded by one that clears the counters.  (us a call, 8192 x 1024 at 16 tokens, split in four: tagged words and their exchange loop alone,
+// a load and up to `splits` contended exchanges, 7.7; raising a tagged word and then adding to it 6.3; one addition to a word of four
+// bytes, with 20 bits for the sum of the epochs, 5.1; this 4.6, half as many counters to a cache line.)
+__host__ __device__ __forceinline__ bool arrive_last(int* counters, int tile, int splits, int epoch)
 {
     if (epoch == 0) {
-        const bool last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1;
+        int* const counter = counters + tile;
+        const bool last    = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1;
         if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return last;
     }
-    const uint32_t one   = ((uint32_t)epoch << kEpochShift) + 1;
-    const uint32_t found = (uint32_t)__hip_atomic_fetch_add(counter, (int)one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t j     = found & ((1u << kEpochShift) - 1);
+    uint64_t* const counter = reinterpret_cast<uint64_t*>(counters) + tile;
+    const uint64_t  one     = (uint64_t)(uint32_t)epoch << 32 | 1;
+    const uint64_t  found   = __hip_atomic_fetch_add(counter, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t  j       = (uint32_t)found;
     if (j < (uint32_t)splits && found == j * one) {
         const bool last = j == (uint32_t)splits - 1;
-        if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (last) __hip_atomic_store(counter, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return last;
     }
-    int* const tagged = counter + kStaticCounters;
+    int* const tagged = counters + kStaticTagged + tile;
     int        seen   = __hip_atomic_load(tagged, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {  // (a failed exchange means that another workgroup has arrived: at most `splits` rounds)
         const int n    = (seen >> kEpochShift) == epoch ? seen & ((1 << kEpochShift) - 1) : 0;
         const int next = n == splits - 1 ? 0 : (epoch << kEpochShift) | (n + 1);
         if (__hip_atomic_compare_exchange_strong(tagged, &seen, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-            if (n == splits - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (n == splits - 1) __hip_atomic_store(counter, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return n == splits - 1;
         }
     }

@@ -85,7 +85,7 @@ struct Scratch {
     int    epoch;  // tag of this launch's counts where the counters are shared, else 0 (arrive_last)
     int    cus;    // compute units of the device that all this is on, which the strips are dealt to and the prices counted in
 };
-constexpr int kEpochShift = 12;  // a counter word: the epoch above, up to 4095 arrivals below
+constexpr int kEpochShift = 12;  // a tagged counter word: the epoch above, up to 4095 arrivals below
 
 // Launches `kernel` and returns this launch's own status.  (The triple-chevron form reports through
 // hipGetLastError, which also returns - and clears - an error some earlier call of the caller left behind.)
@@ -131,6 +131,10 @@ hipError_t algo_launch(int id, int nq, const GemmArgs& a, const Scratch& sc, hip
 // The scratch that lives in a file-scope device array (static_scratch.hip), for callers that cannot
 // allocate: its address on the current device, looked up once per device.
 constexpr size_t kStaticCounters       = 4096;
+// In front of the partial tiles, so many of each (arrive_last): counters of launches made at once, eight bytes each; from int kStaticTagged
+// on, the second ones, for counts that did not start from zero; from int kStaticRecorded on, the counters of launches recorded into a graph.
+constexpr size_t kStaticTagged         = 2 * kStaticCounters;
+constexpr size_t kStaticRecorded       = 3 * kStaticCounters;
 constexpr size_t kStaticWorkspaceBytes = 8u << 20;
 hipError_t static_scratch(Scratch* out);
 // before a launch that uses `n` of its counters: sets the tag, and clears them where the launch is being recorded into a graph

@@ -8,7 +8,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-TAG_SHIFT = 12      # a counter word: the launch's tag above, arrivals below (w4a16_internal.h, kEpochShift)
+TAG_SHIFT = 12      # a tagged counter word: the launch's tag above, arrivals below (w4a16_internal.h, kEpochShift)
 
 
 class Scratch(ctypes.Structure):
@@ -25,14 +25,22 @@ def scratch(lib):
     return s
 
 
-def leave_behind(lib, word):
+def write_counters(lib, words):
+    """All three parts of the counters (w4a16_internal.h, kStaticCounters): eight bytes each of launches made at once, tagged words, and
+    those of recorded launches."""
     s = scratch(lib)
-    words = (ctypes.c_int * s.cnt_len)(*([word] * s.cnt_len))
+    assert len(words) == 4 * s.cnt_len
     torch.cuda.synchronize()
     fn = lib.hipMemcpy
     fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
-    assert fn(s.cnt, words, 4 * s.cnt_len, 1) == 0      # host to device
+    assert fn(s.cnt, (ctypes.c_int * len(words))(*words), 4 * len(words), 1) == 0      # host to device
     torch.cuda.synchronize()
+
+
+def leave_behind(lib, word):
+    """`word` >> TAG_SHIFT: the tag of a launch, and below it how many arrivals of it every counter holds."""
+    n, count = scratch(lib).cnt_len, word & (1 << TAG_SHIFT) - 1
+    write_counters(lib, [count, (word >> TAG_SHIFT) * count] * n + [word] * n + [word] * n)
 
 
 # a batch kernel as column blocks, the same as blocks of some dozen tokens, column blocks, and MFMA tiles; all split K
@@ -93,13 +101,9 @@ def test_second_counters_left_behind(splits_of):
     X, H, E = torch.randn((T, K), device="cuda", generator=gen).half(), *torch.empty((2, T, N), dtype=torch.float16, device="cuda")
     gemm = tm.GemmS4F16()
     gemm.Run(H, A, X, Q, N, T, K, 128)
-    fn = lib.hipMemcpy
-    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
     for first, second in ((0, 3), (3, 0), (3, 3), (1 << 20, -1), (-1, 2 << TAG_SHIFT | 1)):
-        at = scratch(lib)
-        both = (ctypes.c_int * (2 * at.cnt_len))(*([first] * at.cnt_len + [second] * at.cnt_len))
-        torch.cuda.synchronize()
-        assert fn(at.cnt, both, 8 * at.cnt_len, 1) == 0
+        n = scratch(lib).cnt_len
+        write_counters(lib, [first, first] * n + [second] * n + [0] * n)
         for call in range(3):
             E.fill_(float("nan"))
             tm.gemm_static(E, A, X, Q, N, T, K, 128)
