@@ -112,16 +112,10 @@ batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int 
     const int G  = (int)((uint32_t)K / kGroup);
     const int NT = (int)((uint32_t)N / kTileN);
 
-    // Workgroups are dealt round-robin to the 8 XCDs; each gets a contiguous run, the token tiles of a strip next to
-    // each other (they share its weights), the splits of K outermost (each touches its own part of the activations).
-    const uint32_t log_splits = how & 0xff, splits = 1u << log_splits;
-    const uint32_t total      = (strips * tiles_t) << log_splits;
-    uint32_t       id         = blockIdx.x;
-    if (total % 8 == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-    const uint32_t row    = divide_by(id, tiles_t, by_tiles_t);  // of strips, split by split
-    const int      tile_t = (int)(id - row * tiles_t);
-    const uint32_t split  = log_splits ? divide_by(row, strips, by_strips) : 0;
-    const int      strip  = (int)(row - split * strips);
+    const uint32_t   log_splits = how & 0xff, splits = 1u << log_splits;
+    const BatchPlace at = batch_place(blockIdx.x, strips, tiles_t, by_strips, by_tiles_t, log_splits);
+    const int        tile_t = at.tile_t, strip = at.strip;
+    const uint32_t   split = at.split;
     // the last strip may overlap its neighbour: it then leaves the tiles below `first` to it
     const int first = strip * R;
     const int col0  = min(first, NT - R);
@@ -536,9 +530,8 @@ hipError_t batch_launch(const BatchConfig& cf, int nq, const GemmArgs& a, const 
     if (cf.splits > 1 && (sc.ws == nullptr || sc.cnt == nullptr)) return hipErrorInvalidValue;
     const uint32_t strips = (uint32_t)((a.N / kTileN + cf.r - 1) / cf.r), tiles_t = (uint32_t)((a.T + 16 * cf.h - 1) / (16 * cf.h));
     const uint32_t log_splits = (uint32_t)log2_of(cf.splits);
-    const uint64_t rows = (uint64_t)strips << log_splits;
-    BatchArgs      p{reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.N, a.T, a.K, strips, tiles_t, reciprocal(rows, strips),
-                reciprocal(rows * tiles_t, tiles_t), log_splits | (uint32_t)a.epilogue << 8, a.C, a.R, sc.ws, sc.cnt, sc.epoch};
+    BatchArgs      p{reinterpret_cast<const u32x4_t*>(a.A), a.X, a.Q, a.N, a.T, a.K, strips, tiles_t, by_batch_strips(strips, log_splits),
+                by_batch_tiles(strips, tiles_t, log_splits), log_splits | (uint32_t)a.epilogue << 8, a.C, a.R, sc.ws, sc.cnt, sc.epoch};
     switch (nq) {
         case 1: return launch_h<1>(cf.r, cf.h, p, st);
         case 2: return launch_h<2>(cf.r, cf.h, p, st);

@@ -172,11 +172,11 @@ inline uint32_t reciprocal(uint64_t bound, uint32_t d)
 {
     return d == 1 ? 0 : bound * d < (1ull << 32) ? (uint32_t)((1ull << 32) / d) + 1 : 1;
 }
-__device__ __forceinline__ uint32_t divide_by(uint32_t n, uint32_t d, uint32_t reciprocal)
+__host__ __device__ __forceinline__ uint32_t divide_by(uint32_t n, uint32_t d, uint32_t reciprocal)
 {
     if (reciprocal == 0) return n;
     if (reciprocal == 1) return n / d;
-    return __umulhi(n, reciprocal);
+    return (uint32_t)((uint64_t)n * reciprocal >> 32);
 }
 
 // The place of a workgroup of the MFMA tile kernels: which tile, and which quantisation groups of K.  Workgroups are dealt
@@ -190,7 +190,7 @@ struct TilePlace {
 };
 // what the tiles are divided by on the way, for `reciprocal`
 inline uint32_t tile_divisor(int tiles_t, int tiles_n) { return (uint32_t)(tiles_t % 4 == 0 ? tiles_n : tiles_t); }
-__device__ __forceinline__ TilePlace tile_place(int id, int tiles_t, int tiles_n, uint32_t by_divisor, int G, int split, int log_splits)
+__host__ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_t, int tiles_n, uint32_t by_divisor, int G, int split, int log_splits)
 {
     TilePlace p;
     if (tiles_t % 4 == 0) {
@@ -203,8 +203,35 @@ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_t, int tiles_n
         p.tile_t = id - p.tile_n * tiles_t;
     }
     const uint32_t pairs = ((uint32_t)G + 1) / 2;  // (K below 2^31: times eight splits in 32 bits)
-    p.gbeg = min(G, 2 * (int)(pairs * (uint32_t)split >> log_splits));
-    p.gend = min(G, 2 * (int)(pairs * (uint32_t)(split + 1) >> log_splits));
+    const int      from = 2 * (int)(pairs * (uint32_t)split >> log_splits), to = 2 * (int)(pairs * (uint32_t)(split + 1) >> log_splits);
+    p.gbeg = G < from ? G : from;
+    p.gend = G < to ? G : to;
+    return p;
+}
+
+// The place of workgroup `id` of a batch kernel, of `strips` of columns times `tiles_t` blocks of tokens times K splits.  Again each
+// XCD gets a contiguous run, the token tiles of a strip next to each other (they share its weights), the splits of K outermost
+// (each touches its own part of the activations).
+struct BatchPlace {
+    int      tile_t, strip;
+    uint32_t split;
+};
+// their reciprocals: what is divided by `tiles_t` is below all workgroups, what by `strips` below the strips of all splits
+inline uint32_t by_batch_strips(uint32_t strips, uint32_t log_splits) { return reciprocal((uint64_t)strips << log_splits, strips); }
+inline uint32_t by_batch_tiles(uint32_t strips, uint32_t tiles_t, uint32_t log_splits)
+{
+    return reciprocal(((uint64_t)strips << log_splits) * tiles_t, tiles_t);
+}
+__host__ __device__ __forceinline__ BatchPlace batch_place(uint32_t id, uint32_t strips, uint32_t tiles_t, uint32_t by_strips, uint32_t by_tiles_t,
+                                                           uint32_t log_splits)
+{
+    const uint32_t total = (strips * tiles_t) << log_splits;
+    if (total % 8 == 0) id = (id & 7) * (total >> 3) + (id >> 3);
+    BatchPlace     p;
+    const uint32_t row = divide_by(id, tiles_t, by_tiles_t);  // of strips, split by split
+    p.tile_t = (int)(id - row * tiles_t);
+    p.split  = log_splits ? divide_by(row, strips, by_strips) : 0;
+    p.strip  = (int)(row - p.split * strips);
     return p;
 }
 
