@@ -57,7 +57,7 @@ typedef struct w4a16_metric {
 } w4a16_metric;
 
 /* GemmS4F16::GemmS4F16 / ~GemmS4F16 (gemm_s4_f16.h:19-21, gemm_s4_f16.cu:236-252).
- * The handle owns two events and 256 KiB of arrival counters; it binds to the current device.
+ * The handle owns two events and 512 KiB of arrival counters; it binds to the current device.
  * A fixed 64 MiB workspace for split-K partial sums is allocated by the first launch that splits K
  * (some shapes between 17 and 512 tokens, narrow matrices at up to 16) and kept until
  * w4a16_destroy.  That first launch must not be under graph capture: there, a handle that has no

@@ -16,7 +16,7 @@ namespace w4a16 {
 
 namespace {
 
-constexpr size_t kCounterBytes = 4 * kStaticCounters * sizeof(int);
+constexpr size_t kCounterBytes = kStaticCounterInts * sizeof(int);
 constexpr size_t kStaticBytes  = kCounterBytes + kStaticWorkspaceBytes;
 constexpr int    kMaxDevices   = 64;
 
@@ -82,7 +82,7 @@ hipError_t prepare_static_counters(Scratch* sc, int n, hipStream_t st)
     if (cs == hipStreamCaptureStatusNone) return hipSuccess;
     sc->epoch = 0;
     sc->cnt += kStaticRecorded;
-    n = std::min(n, sc->cnt_len);
+    n = 2 * std::min(n, sc->cnt_len);  // (eight bytes each)
     return launch_kernel(fill_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, st, sc->cnt, n);
 }
 

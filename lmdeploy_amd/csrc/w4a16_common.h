@@ -236,9 +236,9 @@ __host__ __device__ __forceinline__ BatchPlace batch_place(uint32_t id, uint32_t
 }
 
 // Split K: a workgroup announces that its partial tile is complete; true for the last of `splits`, which leaves the counter
-// at zero for the next launch.  epoch 0: the counters belong to a handle, which nobody else touches, or were cleared right before
-// this launch.  Otherwise they are shared by every caller on the GPU, and launches that overlapped against the rules may have left
-// anything in them.  Every arrival then adds one, and the launch's epoch in the upper half of the word: what d arrivals of other
+// at zero for the next launch.  Counters are eight bytes each (`counters`: in ints).  epoch 0: they belong to a handle, which nobody else
+// touches, or were cleared right before this launch.  Otherwise they are shared by every caller on the GPU, and launches that overlapped
+// against the rules may have left anything in them.  Every arrival adds one, and the launch's epoch in the upper half of the word: what d arrivals of other
 // launches left is taken for this launch's own only if their epochs add up to d times its own.  Those of one launch do so when
 // the epochs have come round (2^19 - 1 launches), those of several also if one of them has a higher epoch than this launch and their mean is
 // its own.  The sum is exact: d below the splits, at most 4095, and 19 bits of epoch.  Where the count did not start from zero, no
@@ -246,20 +246,16 @@ __host__ __device__ __forceinline__ BatchPlace batch_place(uint32_t id, uint32_t
 // counts they hold; the last one clears both, so that one misuse does not spoil the launches after it and none of them has to be
 // preceded by one that clears the counters.  (us a call, 8192 x 1024 at 16 tokens, split in four: tagged words and their exchange loop alone,
 // a load and up to `splits` contended exchanges, 7.7; raising a tagged word and then adding to it 6.3; one addition to a word of four
-// bytes, with 20 bits for the sum of the epochs, 5.1; this 4.6, half as many counters to a cache line.)
+// bytes, with 20 bits for the sum of the epochs, 5.1; this 4.6, half as many counters to a cache line.  All kinds of counters go
+// one way, for every instruction here comes with each kernel: with a way of their own for handles the 14 KB of a batch kernel had 140 bytes more, and
+// a chain of eight launches at 48 tokens took 0.9 % longer.)
 __host__ __device__ __forceinline__ bool arrive_last(int* counters, int tile, int splits, int epoch)
 {
-    if (epoch == 0) {
-        int* const counter = counters + tile;
-        const bool last    = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1;
-        if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return last;
-    }
     uint64_t* const counter = reinterpret_cast<uint64_t*>(counters) + tile;
     const uint64_t  one     = (uint64_t)(uint32_t)epoch << 32 | 1;
     const uint64_t  found   = __hip_atomic_fetch_add(counter, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t  j       = (uint32_t)found;
-    if (j < (uint32_t)splits && found == j * one) {
+    if (__builtin_expect(epoch == 0 || (j < (uint32_t)splits && (uint32_t)(found >> 32) == j * (uint32_t)epoch), 1)) {
         const bool last = j == (uint32_t)splits - 1;
         if (last) __hip_atomic_store(counter, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return last;

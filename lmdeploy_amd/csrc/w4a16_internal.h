@@ -80,8 +80,8 @@ constexpr int    kCounters       = 1 << 16;
 struct Scratch {
     float* ws;
     size_t ws_bytes;
-    int*   cnt;
-    int    cnt_len;
+    int*   cnt;      // eight bytes each
+    int    cnt_len;  // counters
     int    epoch;  // tag of this launch's counts where the counters are shared, else 0 (arrive_last)
     int    cus;    // compute units of the device that all this is on, which the strips are dealt to and the prices counted in
 };
@@ -132,9 +132,11 @@ hipError_t algo_launch(int id, int nq, const GemmArgs& a, const Scratch& sc, hip
 // allocate: its address on the current device, looked up once per device.
 constexpr size_t kStaticCounters       = 4096;
 // In front of the partial tiles, so many of each (arrive_last): counters of launches made at once, eight bytes each; from int kStaticTagged
-// on, the second ones, for counts that did not start from zero; from int kStaticRecorded on, the counters of launches recorded into a graph.
+// on, the second ones, four bytes, for counts that did not start from zero; from int kStaticRecorded on, eight bytes, those of launches
+// recorded into a graph.
 constexpr size_t kStaticTagged         = 2 * kStaticCounters;
 constexpr size_t kStaticRecorded       = 3 * kStaticCounters;
+constexpr size_t kStaticCounterInts    = 5 * kStaticCounters;
 constexpr size_t kStaticWorkspaceBytes = 8u << 20;
 hipError_t static_scratch(Scratch* out);
 // before a launch that uses `n` of its counters: sets the tag, and clears them where the launch is being recorded into a graph

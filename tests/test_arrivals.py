@@ -38,7 +38,7 @@ def test_arrivals_of_one_launch_after_another(lib, splits):
     for epoch in (1, 2, 3, 12345, PERIOD, 1):
         assert c.arrive(splits, epoch) == once(splits) and c.clean()
     for _ in range(3):
-        assert c.arrive(splits, 0) == once(splits) and c.words[5] == 0      # a handle's counters
+        assert c.arrive(splits, 0) == once(splits) and c.clean()      # a handle's counters
 
 
 # A launch leaves fewer than its splits.  1 << 18, 1 << 13 and the like: where d times one tag and d times another agree in 20 bits.

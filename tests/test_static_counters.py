@@ -26,10 +26,10 @@ def scratch(lib):
 
 
 def write_counters(lib, words):
-    """All three parts of the counters (w4a16_internal.h, kStaticCounters): eight bytes each of launches made at once, tagged words, and
-    those of recorded launches."""
+    """All three parts of the counters (w4a16_internal.h, kStaticCounters): eight bytes each of launches made at once, tagged words of
+    four, and eight each of recorded launches."""
     s = scratch(lib)
-    assert len(words) == 4 * s.cnt_len
+    assert len(words) == 5 * s.cnt_len
     torch.cuda.synchronize()
     fn = lib.hipMemcpy
     fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
@@ -40,7 +40,7 @@ def write_counters(lib, words):
 def leave_behind(lib, word):
     """`word` >> TAG_SHIFT: the tag of a launch, and below it how many arrivals of it every counter holds."""
     n, count = scratch(lib).cnt_len, word & (1 << TAG_SHIFT) - 1
-    write_counters(lib, [count, (word >> TAG_SHIFT) * count] * n + [word] * n + [word] * n)
+    write_counters(lib, [count, (word >> TAG_SHIFT) * count] * n + [word] * n + [word] * 2 * n)
 
 
 # a batch kernel as column blocks, the same as blocks of some dozen tokens, column blocks, and MFMA tiles; all split K
@@ -103,7 +103,7 @@ def test_second_counters_left_behind(splits_of):
     gemm.Run(H, A, X, Q, N, T, K, 128)
     for first, second in ((0, 3), (3, 0), (3, 3), (1 << 20, -1), (-1, 2 << TAG_SHIFT | 1)):
         n = scratch(lib).cnt_len
-        write_counters(lib, [first, first] * n + [second] * n + [0] * n)
+        write_counters(lib, [first, first] * n + [second] * n + [0] * 2 * n)
         for call in range(3):
             E.fill_(float("nan"))
             tm.gemm_static(E, A, X, Q, N, T, K, 128)
