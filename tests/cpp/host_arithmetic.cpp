@@ -1,4 +1,5 @@
-// The whole-number arithmetic of csrc/w4a16_common.h that kernels and host share, as functions to call from a test.
+// The whole-number arithmetic of csrc/w4a16_common.h that kernels and host share, as functions to call from a test, and what
+// the members of a configuration are.
 #include "../../lmdeploy_amd/csrc/w4a16_common.h"
 
 extern "C" int arrive(int* counters, int tile, int splits, int epoch) { return w4a16::arrive_last(counters, tile, splits, epoch); }
@@ -19,4 +20,10 @@ extern "C" void batch_at(unsigned id, unsigned strips, unsigned tiles_t, int spl
     const unsigned          z = (unsigned)w4a16::log2_of(splits);
     const w4a16::BatchPlace p = w4a16::batch_place(id, strips, tiles_t, w4a16::by_batch_strips(strips, z), w4a16::by_batch_tiles(strips, tiles_t, z), z);
     out[0] = p.tile_t, out[1] = p.strip, out[2] = (int)p.split;
+}
+
+extern "C" void describe(const w4a16::Algo* a, int* out)
+{
+    out[0] = a->family == w4a16::kBatch ? 'b' : a->family == w4a16::kStrip ? 's' : 't';
+    out[1] = a->tile_n, out[2] = a->tile_t, out[3] = a->bc.splits;
 }
