@@ -68,7 +68,7 @@ struct Algo {
     TileConfig   tc;       // tile only
     int          depth;    // K steps come in multiples of this
     int          resident; // workgroups that fit a CU
-    Cost         cost, few;  // few: up to 128 tokens
+    Cost         cost, few;  // few: of batch kernels at up to 128 tokens, 32 with group sizes 64 and 32 (pick_by_cost)
 };
 
 // Scratch of the split-K kernels: fp32 partial tiles and arrival counters.  A handle's scratch has
