@@ -182,6 +182,15 @@ batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int 
 #pragma unroll
         for (int h = 0; h < H; ++h) acc[r][h] = float4_t{0.f, 0.f, 0.f, 0.f};
 
+    // Four quantisation groups per tile: its words, a lane row for each group, are spread over the rows once, in the first half, a scale that
+    // reads as zero being cleared before that for all of them.  (Beside two waves' MFMAs there is little room for vector instructions: 22
+    // a tile and half went into its words, now 10.  Group size 32, cold weights, spread and taken apart in either half -> once, us:
+    // 11008 x 4096 at 32 / 100 tokens 14.0 -> 13.3 / 26.1 -> 25.2, 4096 x 4096 at 24 / 100 6.64 -> 6.42 / 11.7 -> 11.4, 4096 x 22016 at 48 22.6
+    // -> 22.2, 4096 x 12288 at 48 13.4 -> 13.2.  Blocks of 4 x 5 and 6 x 4, whose registers are all in use, gain nothing (300 tokens of a 7B layer 173.5
+    // and 174.4) and keep the other way, and so do two groups or one, where there is less to save and 6 x 4 spills.)
+    constexpr bool kOnce = NQ == 4 && R * H < 20;
+    uint32_t       late[R][2];  // of the second half's groups
+    constexpr int kSubs = NQ == 4 ? 2 : 1;  // quantisation groups in half a tile
     // Half a group: two chunks of 32 rows of K.  All fragments are read first: the patch is then free, and its next rows
     // are requested before the arithmetic, so that both patches of a wave are in flight nearly all the time (what the
     // vector memory path of a CU needs to stay busy is about 130 KiB in flight).
@@ -191,17 +200,41 @@ batch_kernel(const u32x4_t* A, const uint16_t* X, const uint32_t* Q, int N, int 
         static_for<0, 2>([&](auto j) { static_for<0, H>([&](auto h) { lds_read128<hf * kPatch + h * 2048>(xf[j][h], xr[j]); }); });
         // the scales of a tile, as fp32, and what the unpacked nibbles carry beside q - z: of every quantisation group in
         // this half
-        constexpr int kSubs = NQ == 4 ? 2 : 1;
         float         sf[kSubs];
         half2_t       z1024[kSubs], z64[kSubs];
         auto          words = [&](int r) {
-            uint32_t q[NQ];
-            spread_q<NQ>(s.q[r], q);
+            if constexpr (!kOnce) {
+                uint32_t q[NQ];
+                spread_q<NQ>(s.q[r], q);
 #pragma unroll
-            for (int u = 0; u < kSubs; ++u) {
-                half_t sc;
-                split_q(q[NQ == 1 ? 0 : NQ == 2 ? hf : 2 * hf + u], z1024[u], z64[u], sc);
-                sf[u] = (float)sc;
+                for (int u = 0; u < kSubs; ++u) {
+                    half_t sc;
+                    split_q(q[NQ == 1 ? 0 : NQ == 2 ? hf : 2 * hf + u], z1024[u], z64[u], sc);
+                    sf[u] = (float)sc;
+                }
+            }
+            else {
+                uint32_t q[2];
+                if constexpr (hf == 0) {
+                    uint32_t all[4];
+                    spread_q<4>(scale_is_normal(s.q[r]) ? s.q[r] : s.q[r] & 0xffffu, all);
+                    q[0] = all[0], q[1] = all[1];
+                    late[r][0] = all[2], late[r][1] = all[3];
+                }
+                else {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        q[u] = late[r][u];
+                        asm volatile("" : "+v"(q[u]));  // (what is made of it is made here: the first half has no registers for it)
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const half2_t h = as_half2(q[u]), z = as_half2(((q[u] >> 4) & 0xfu) | 0x6400u);
+                    z64[u]   = half2_t{h[0], h[0]};
+                    z1024[u] = half2_t{z[0], z[0]};
+                    sf[u]    = (float)h[1];
+                }
             }
         };
         auto integers = [&](int r, auto j) {

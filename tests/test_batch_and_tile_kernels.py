@@ -64,6 +64,29 @@ def test_group_sizes_64_and_32_on_both_sides_of_every_hand_over(tm, gs, K, N):
 
 
 @pytest.mark.parametrize("gs", [64, 32])
+@pytest.mark.parametrize("T,N", [(9, 272), (17, 272), (33, 1088), (48, 4096), (48, 16384), (65, 4096), (100, 4096), (300, 4096)])
+def test_subnormal_scales_of_small_groups(tm, gs, T, N):
+    """A subnormal scale reads as zero whichever of a weight tile's groups it belongs to, in blocks of every width."""
+    K   = 640
+    gen = torch.Generator(device="cuda").manual_seed(T + N + gs)
+    words = lambda *size: torch.randint(-2 ** 31, 2 ** 31, size, dtype=torch.int32, device="cuda", generator=gen)
+    s = (torch.randn((K // gs, N), device="cuda", generator=gen).abs() * 0.01 + 1e-3).half()
+    for col in range(7):  # another group in every seventh column, and the smallest normal scale beside them
+        s[col % (128 // gs)::128 // gs, col::7] = 2.0 ** -15 if col < 6 else 2.0 ** -14
+    qw = words(K, N // 8)
+    A, Q = torch.empty_like(qw), torch.empty_like(s, dtype=torch.int32)
+    tm.convert_s4_k_m8(A, Q, s, qw, s, words(K // gs, N // 8), N, K, gs)
+    W = tm.dequantize_repacked(A, Q, N, K, gs).float()
+    assert (W.view(K // gs, gs, N)[0, :, 0] == 0).all()
+    X = (1000 * torch.randn((T, K), device="cuda", generator=gen)).half()  # (a product that is not left out would show)
+    want = X.float() @ W
+    allowed = HALF_ULP * want.abs() + (HALF_ULP + HALF_ULP / 4) * (X.float().abs() @ W.abs())
+    C = torch.full((T, N), float("nan"), dtype=torch.float16, device="cuda")
+    tm.GemmS4F16().Run(C, A, X, Q, N, T, K, gs)
+    assert ((C.float() - want).abs() <= allowed).all()
+
+
+@pytest.mark.parametrize("gs", [64, 32])
 @pytest.mark.parametrize("K,N", [(4096 + 128, 272)] + [(384, 4096 * w - 896) for w in range(2, 9)] + [(128, 4096 * 9)])
 def test_strips_of_every_width_with_small_groups(tm, gs, K, N):
     """One tile with sixteen waves, strips of two to eight tiles next to narrower ones, and several strips in turn."""
