@@ -52,3 +52,8 @@ def test_blocks_of_one_token_tile_end_where_they_are_priced(chosen, nq):
     assert chosen(4096, 4096, 24, nq) == (BATCH, 32, 16, 1)
     assert all(chosen(N, K, T, nq)[2] != 16 for N in (1024, 4096, 5120) for K in (1024, 4096, 11008) for T in (97, 100, 128, 129, 300)
                if chosen(N, K, T, nq)[0] == BATCH)
+
+
+@pytest.mark.parametrize("N,K,T", [(3456, 4608, 351), (1728, 8320, 925), (9984, 2176, 118), (4480, 5120, 247)])
+def test_tiles_of_64_by_64_are_not_taken_where_they_fill_the_chip_twice(chosen, N, K, T):
+    assert chosen(N, K, T)[1:3] != (64, 64) or chosen(N, K, T)[0] == BATCH
